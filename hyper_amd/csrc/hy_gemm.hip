@@ -386,14 +386,18 @@ template <> struct Raw<IQ4_NL> {
     __device__ __forceinline__ float fold(int si, int) const { return (float) si; }
 };
 // Q8_0 weights (8 blocks of 34 B per 256 values, Q8_0 activations): chunk c = block c; lane values 8 q .. + 7 are
-// qs[8 q ..] of block c as they are (int8); block c's qs sit at 34 c + 2 (2 mod 4 for even c, where the 8-byte read
-// takes 2 bytes of block c + 1, c < 7); every block folds on its own, as IQ4_NL's.
+// qs[8 q ..] of block c as they are (int8); every block folds on its own, as IQ4_NL's.  The spans are 16-byte aligned,
+// so block c's qs (34 c + 2) are 2 mod 4 for even c, read by ld8_2a whose 12 bytes end at most at blk + 239, and
+// dword-aligned for odd c, read as they are: block 7's last 8 bytes end the span, and of the last row the allocation.
 template <> struct Raw<Q8_0> {
     static constexpr bool mins = false, g16 = false, per_chunk = true;
     uint2 qv[8]; uint32_t dd[4];
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) qv[c] = ld8_2a(blk + 34 * c + 2 + 8 * q);
+        for (int c = 0; c < 8; ++c) {
+            const uint8_t *p = blk + 34 * c + 2 + 8 * q;
+            qv[c] = (c & 1) ? *(const uint2 *) p : ld8_2a(p);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) dd[i] = (uint32_t) ld_u16(blk + 68 * i) | ((uint32_t) ld_u16(blk + 68 * i + 34) << 16);
     }
