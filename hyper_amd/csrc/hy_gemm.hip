@@ -758,6 +758,93 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
     asm volatile("");   // keeps the tile-count variants from being merged (which moved the accumulators to memory)
 }
 
+// IQ2_XS step on the 16x16x64 MFMA.  Lane quarter q's 16 values of MFMA j (64 j + 16 q ..) are scale group 4 j + q: the
+// two 8-groups of the 32-bit word qs[8 j + 2 q], qs[8 j + 2 q + 1] (9 bits of grid row, 7 of sign index each), scale
+// s = 2 nibble + 1 in 1 .. 31.  The codebook has three levels, 8 = 8 1 + 9 0, 25 = 8 2 + 9 1 and 43 = 8 2 + 9 3, so
+// B = sign s level splits into two int8 planes, B = 8 P + Q with P = sign s {1, 2, 2}, |P| <= 62, and Q = sign s {0, 1, 3},
+// |Q| <= 93: sum_g s_g dot_g = 8 X.P + 9 X.Q exactly.  A plane's byte is one of six per scale group (level, sign), held
+// in two registers, and v_perm picks four at a time: the LDS tables give each 8-group's levels and signs as nibbles
+// (iq2_sel_table: entry g the levels of row g, entry 512 + i the signs of sign index i in bit 2 of each nibble; value v
+// of the 8-group in byte v % 4, nibble v / 4), OR-ed into the selectors.  It replaced the generic step (two masked
+// 16x16x32 MFMAs a 32-value chunk, eight 24-bit multiply-adds an output column, 8-byte codebook and sign rows): the
+// 2048-token, 384-expert layer of d 7168, ff 2048, top-6: gate/up 3.95 -> 2.15 ms, down 2.05 -> 1.04 ms.  Bound by VALU
+// issue (75 % of the cycles at 16 waves, 290 instructions a wave and step; LDS 50 %, MFMA 20 %).
+constexpr int IQ2_SEL = 512 + 128;
+__device__ __forceinline__ void iq2_sel_table(uint32_t *sel) {
+    for (int i = threadIdx.x; i < IQ2_SEL; i += blockDim.x) {
+        uint32_t v = 0, c = i < 512 ? c_iq2xs_code[i] : ksign((uint32_t) i - 512);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t n = i < 512 ? c % 3 : (c & 1) << 2;
+            c = i < 512 ? c / 3 : c >> 1;
+            v |= n << (8 * (j & 3) + 4 * (j >> 2));
+        }
+        sel[i] = v;
+    }
+}
+// 4 bytes at p, which is 2-byte aligned (sb = p & 3 is 0 or 2): two aligned dwords from p - sb, joined.  (One unaligned
+// LDS read costs about 60 cycles of the CU's LDS pipe: SQ_LDS_UNALIGNED_STALL.)
+__device__ __forceinline__ uint32_t ld4_u2(const uint8_t *p, uint32_t sb) {
+    const uint32_t *w = (const uint32_t *) (p - sb);
+    return __builtin_amdgcn_alignbyte(w[1], w[0], sb);
+}
+template <int NT, int T0, bool FIRST>
+__device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as, const float *yd, const uint32_t *sel, float (&acc)[GM_TILES][4]) {
+    // the tiles past NT hold nothing this item reads: marking them redefined frees their registers (as in step_q4k)
+#pragma unroll
+    for (int t = T0 + NT; t < GM_TILES; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
+    const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
+    const uint8_t *blk = wt0 + rr * block_bytes(IQ2_XS);
+    const uint32_t al = 2u * (uint32_t) (~rr & 1);   // the tile starts dword-aligned: qs and scales of even rows are 2 mod 4
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = ld4_u2(blk + 2 + 16 * j + 4 * q, al);
+    const uint32_t sc0 = ld4_u2(blk + 66, al) >> (4 * q), sc1 = ld4_u2(blk + 70, al) >> (4 * q);   // group 4 j + q: nibble 0 / 4
+    const float d = h2f(ld_u16(blk)) * 0.125f;
+    const int8_t *arow = as + rr * 256;
+    const v4i z = {0, 0, 0, 0};
+    v4i dp[NT], dq[NT];
+    uint32_t ga[4], sa[4], gb[4], sb[4];   // every lookup of the step goes out before the first MFMA
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        ga[j] = sel[__builtin_amdgcn_ubfe(w[j], 0, 9)];
+        sa[j] = sel[512 + __builtin_amdgcn_ubfe(w[j], 9, 7)];
+        gb[j] = sel[__builtin_amdgcn_ubfe(w[j], 16, 9)];
+        sb[j] = sel[512 + (w[j] >> 25)];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t ca = ga[j] | sa[j], cb = gb[j] | sb[j];
+        const uint32_t s = 2 * (((j < 2 ? sc0 : sc1) >> (16 * (j & 1))) & 15) + 1, s2 = s | (s << 16);
+        const uint32_t Pp = (uint32_t) mul_bytes(0x00020201u, s2), Qp = (uint32_t) mul_bytes(0x00030100u, s2);
+        const uint32_t Pn = (Pp ^ 0x00FFFFFFu) + 0x00010101u, Qn = (Qp ^ 0x00FFFF00u) + 0x00010100u;   // the negated bytes
+        const uint32_t i0 = ca & 0x07070707u, i1 = (ca >> 4) & 0x07070707u, i2 = cb & 0x07070707u, i3 = (cb >> 4) & 0x07070707u;
+        const v4i BP = {(int) __builtin_amdgcn_perm(Pn, Pp, i0), (int) __builtin_amdgcn_perm(Pn, Pp, i1),
+                        (int) __builtin_amdgcn_perm(Pn, Pp, i2), (int) __builtin_amdgcn_perm(Pn, Pp, i3)};
+        const v4i BQ = {(int) __builtin_amdgcn_perm(Qn, Qp, i0), (int) __builtin_amdgcn_perm(Qn, Qp, i1),
+                        (int) __builtin_amdgcn_perm(Qn, Qp, i2), (int) __builtin_amdgcn_perm(Qn, Qp, i3)};
+        const int po = 16 * ((4 * j + q) ^ rr);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const v4i A = *(const v4i *) (arow + (T0 + t) * 16 * 256 + po);
+            dp[t] = mfma64(A, BP, j ? dp[t] : z);
+            dq[t] = mfma64(A, BQ, j ? dq[t] : z);
+            asm volatile("");   // a scheduling-region boundary: operands are not hoisted across tiles (register pressure)
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int si = ((dp[t][v] + dq[t][v]) << 3) + dq[t][v];
+            acc[T0 + t][v] = __builtin_fmaf(yd[(T0 + t) * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[T0 + t][v]);
+        }
+    }
+    asm volatile("");   // keeps the tile-count variants from being merged
+}
+
 __host__ __device__ constexpr int xcd_gcd8(int n) { return (n & 7) == 0 ? 8 : (n & 3) == 0 ? 4 : (n & 1) == 0 ? 2 : 1; }
 
 
@@ -778,7 +865,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     __shared__ int s_item[C::ITEMS][3];                  // first pair in order, tokens, weight slot
     __shared__ int s_pair[C::ITEMS][GM_TOK];             // pair index of each token of the segment's items
     __shared__ float s_wt[GU ? 1 : C::ITEMS][GM_TOK];    // down: their route weights
-    __shared__ uint2 grid[iq2_lds(T)];
+    __shared__ uint2 grid[T == IQ2_XS ? IQ2_SEL / 2 : iq2_lds(T)];   // the codebook (IQ2_XS: its selector table)
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, rr = lane & 15, q = lane >> 4;
     const int na = order_n[1];
     // ---- items.  Expert group g (cnt tokens) owns ceil(cnt / 64) items: full ones of 4 token tiles and a last one of
@@ -809,7 +896,8 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
         uint64_t ex = base + inc - loc;
 #pragma unroll
         for (int i = 0; i < C::PER; ++i) { s_scan[C::PER * tid + i] = ex; ex += c2[i]; }
-        if constexpr (iq2_type(T)) expand_iq2_grid<T>(grid);
+        if constexpr (T == IQ2_XS) iq2_sel_table((uint32_t *) grid);
+        else if constexpr (iq2_type(T)) expand_iq2_grid<T>(grid);
         __syncthreads();
     }
     uint64_t tot = 0;
@@ -976,6 +1064,24 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     default: step_q6k<4, 0, false>(wt, as, yd, acc); break;
                     }
                 }
+            } else if constexpr (T == IQ2_XS) {
+                const uint8_t *wt = stage_w(stage) + wave * C::TB;
+                const uint32_t *sel = (const uint32_t *) grid;
+                if (b == 0) {
+                    switch (ntile) {
+                    case 1: step_iq2xs<1, 0, true>(wt, as, yd, sel, acc); break;
+                    case 2: step_iq2xs<2, 0, true>(wt, as, yd, sel, acc); break;
+                    case 3: step_iq2xs<3, 0, true>(wt, as, yd, sel, acc); break;
+                    default: step_iq2xs<4, 0, true>(wt, as, yd, sel, acc); break;
+                    }
+                } else {
+                    switch (ntile) {
+                    case 1: step_iq2xs<1, 0, false>(wt, as, yd, sel, acc); break;
+                    case 2: step_iq2xs<2, 0, false>(wt, as, yd, sel, acc); break;
+                    case 3: step_iq2xs<3, 0, false>(wt, as, yd, sel, acc); break;
+                    default: step_iq2xs<4, 0, false>(wt, as, yd, sel, acc); break;
+                    }
+                }
             } else {
             Raw<T> wr;
             wr.load(stage_w(stage) + wave * C::TB + rr * C::BB, q);
@@ -1051,7 +1157,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     for (int r = lane; r < OR; r += 64) store_f32(o + r, GU ? hy_swiglu(so[r], su[r], m.clamp) : wt * so[r]);
                 }
             }
-            if constexpr (T != Q4_K && T != Q6_K) {   // (the Q4_K / Q6_K steps start the next item's sums themselves)
+            if constexpr (T != Q4_K && T != Q6_K && T != IQ2_XS) {   // (those types' steps start the next item's sums themselves)
 #pragma unroll
                 for (int tile = 0; tile < GM_TILES; ++tile)
 #pragma unroll
@@ -1347,7 +1453,7 @@ int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs,
         return check_launch("hy_moe_gemm_gate_up");
     }
     HY_GEMM_SWITCH(m.tg, {
-        constexpr int W = 8, B = g5_blocks<TT, true>();
+        constexpr int W = TT == IQ2_XS ? 16 : 8, B = g5_blocks<TT, true>();
         const int rb = m.ff / (8 * W);   // 8 W output rows a block
         dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, B == 1));   // two blocks a CU: every slot counts
         hipLaunchKernelGGL((k_gemm<TT, true, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
@@ -1370,7 +1476,7 @@ int launch_gemm_down(const hy_moe_dev &m, const void *hq, int n_pairs, const int
     if ((size_t) n_pairs * (m.ff / 256) * Q8K_BYTES >= (1ull << 32)) { set_error("hy_moe_gemm_down: activations of 4 GB or more"); return HY_EBAD_SHAPE; }
     if (max_items(n_pairs, max_active) >= GM_MAX_ITEMS) { set_error("hy_moe_gemm_down: %d pairs make more than %d work items", n_pairs, GM_MAX_ITEMS - 1); return HY_EBAD_SHAPE; }
     HY_GEMM_SWITCH(m.td, {
-        constexpr int W = TT == Q6_K ? 16 : 8, B = g5_blocks<TT, false>();   // Q6_K: 16 waves (fits 128 registers)
+        constexpr int W = TT == Q6_K || TT == IQ2_XS ? 16 : 8, B = g5_blocks<TT, false>();   // 16 waves where the step fits 128 registers
         const int rb = m.n / (16 * W);   // 16 W output rows a block
         dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, true));
         hipLaunchKernelGGL((k_gemm<TT, false, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) hq, div_mul_of(1), order, order_n, egrp, wts, y);
