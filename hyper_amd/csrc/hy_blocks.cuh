@@ -21,18 +21,19 @@ __device__ __forceinline__ void scale_min_k4(uint32_t s0, uint32_t s1, uint32_t 
     if (j < 4) { sc = byte_of(v, j) & 63; mn = byte_of(v, j + 4) & 63; }
     else { sc = (byte_of(v, j + 4) & 0xF) | ((byte_of(v, j - 4) >> 6) << 4); mn = (byte_of(v, j + 4) >> 4) | ((byte_of(v, j) >> 6) << 4); }
 }
-// four packed nibble indices (bytes 0..15) -> entries of a 16-byte int8 codebook T0..T3 as packed int8
-__device__ __forceinline__ uint32_t kv16(uint32_t idx, uint32_t T0, uint32_t T1, uint32_t T2, uint32_t T3) {
-    const uint32_t sel = idx & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
-    // 0xFF in the bytes whose index is 8..15: selector idx >> 1 picks a byte of 0xFFFFFFFF (4..7) or of 0 (0..3)
-    const uint32_t m = __builtin_amdgcn_perm(0xFFFFFFFFu, 0u, (idx >> 1) & 0x07070707u);
-    return (hi & m) | (lo & ~m);
+// four packed nibble indices (bytes 0..15) -> entries of a 16-byte int8 codebook as packed int8, in four operations:
+// v_perm picks bytes 0..7 of a table by a selector 0..7, and for 8..11 gives the sign of byte 1, 3, 5, 7 spread over the
+// byte, for 12 gives 0x00, for 13..15 0xFF.  So the low half L looked up by idx and the high half H by idx ^ 8 each add a
+// known byte in the other's range, and the tables hold the codebook XOR-ed with that byte: L[i] = cb[i] ^ g(H, i),
+// H[i] = cb[8 + i] ^ g(L, i), g(T, i) = T's byte for selector 8 + i.  (Selecting between the halves with a mask from
+// bit 3 took seven operations; the decode kernels of these types are bound by VALU issue.)
+__device__ __forceinline__ uint32_t kv16(uint32_t idx, uint32_t L0, uint32_t L1, uint32_t H0, uint32_t H1) {
+    return __builtin_amdgcn_perm(L1, L0, idx) ^ __builtin_amdgcn_perm(H1, H0, idx ^ 0x08080808u);
 }
 // the IQ4_NL codebook (bytes: -127 -104 -83 -65 | -49 -35 -22 -10 | 1 13 25 38 | 53 69 89 113)
-__device__ __forceinline__ uint32_t kv4(uint32_t idx) { return kv16(idx, 0xBFAD9881u, 0xF6EADDCFu, 0x26190D01u, 0x71594535u); }
+__device__ __forceinline__ uint32_t kv4(uint32_t idx) { return kv16(idx, 0x40529881u, 0x091522CFu, 0x26190DFEu, 0x8EA6BA35u); }
 // the MXFP4 codebook, E2M1 values doubled (src/kernels4.cu:551; bytes: 0 1 2 3 | 4 6 8 12 | 0 -1 -2 -3 | -4 -6 -8 -12)
-__device__ __forceinline__ uint32_t kvfp4(uint32_t idx) { return kv16(idx, 0x03020100u, 0x0C080604u, 0xFDFEFF00u, 0xF4F8FAFCu); }
+__device__ __forceinline__ uint32_t kvfp4(uint32_t idx) { return kv16(idx, 0x030201FFu, 0xF3F7F904u, 0x0201FF00u, 0x0B0705FCu); }
 // IQ2 signs: 8 sign bits -> two words whose bytes are 0xFF where negated; value = (g ^ M) + (M & 1)
 __device__ __forceinline__ uint32_t spread4(uint32_t b4) { return (b4 * 0x00204081u) & 0x01010101u; }
 // 0xFC in the bytes holding 1 (the others 0): OR-ed onto a 2-bit value it makes the int8 value - 4
