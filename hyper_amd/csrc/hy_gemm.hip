@@ -575,25 +575,40 @@ __device__ __forceinline__ void store_f32(float *g, float v) { asm volatile("glo
 // a store still in flight only makes a later wait stricter (loads cannot overtake the loads before them).
 // Geometry of the stream kernel for weight type T, W waves (8 or 16) per block and B blocks per CU (1 or 2): the
 // stages get what is left of the CU's 160 KB LDS after the item tables.
+//
+// Types with Q8_0 activations (A0): their 34-byte blocks are 2-byte aligned, and an LDS read off its natural alignment
+// costs about 60 cycles of the CU's LDS pipe, so a span's rows (272 bytes each) land as they are in a buffer of their own
+// and are copied into an aligned one (Relay) a step before they are used.  Two weight stages, two raw and two aligned
+// activation buffers: step s computes from weights s and aligned rows s while weights s + 1 and raw rows s + 2 are in
+// flight and rows s + 1 are copied; every wait is for all of a wave's DMAs.  509 tokens, 288 experts, d 4096, ff 1536,
+// top-8 in IQ4_NL: the layer call 2270 us with both operands staged through registers (k_gemm_nl: one step ahead, 4
+// waves, a 7-operation codebook and a 3-operation fold) -> 1038 us; bound by VALU issue (77 % of the cycles).  8 waves
+// of 32 rows instead of 16 of 16 share each activation read but hide less latency: 1196 against 1115 us at the time.
 template <int T, int W, int B> struct G5 {
+    static constexpr bool A0 = vec_dot_type(T) == Q8_0;
     static constexpr int WAVES = W, THREADS = 64 * W, ROWS = 16 * W;   // a wave owns 16 weight rows
     static constexpr int HALF = W / 2;                          // gate/up: waves 0 .. HALF - 1 in gate, the rest in up
     static constexpr int TPW = GM_TOK / W;                      // activation rows each wave fetches per step
-    static constexpr int NA = TPW / 4;                          // their 1 KB DMA instructions
+    static constexpr int AROW = A0 ? 8 * Q8_0_BYTES : Q8K_BYTES;   // activation bytes of a row and span
+    static constexpr int NA = A0 ? (TPW * 17 + 63) / 64 : TPW / 4;  // their DMA instructions (1 KB; A0: 17 16-byte pieces a row)
     static constexpr int PER = 1024 / THREADS;                  // expert groups per thread in the item scan
     static constexpr int ITEMS = B == 1 ? 16 : 8;               // items per segment (their tables live in LDS)
     static constexpr int LDS_STAGES = B == 1 ? 150 * 1024 : 72 * 1024;
-    static constexpr int BB = block_bytes(T);                   // weight bytes per row and 256 values
+    static constexpr int BB = span_bytes(T);                    // weight bytes per row and 256 values
     static constexpr int TB = 16 * BB;                          // one wave's 16-row tile of a span
     static constexpr int WB = W * TB;                           // weights of a stage
-    static constexpr int AB = GM_TOK * 256;                     // activation values of a stage (64 rows of 256)
-    static constexpr int SB = WB + AB + 4 * GM_TOK;             // + the rows' Q8_K d
-    static constexpr int D = 4 * SB <= LDS_STAGES ? 4 : 3 * SB <= LDS_STAGES ? 3 : 2;   // stages
+    static constexpr int AB = A0 ? 0 : GM_TOK * 256;            // activation values of a stage (64 rows of 256)
+    static constexpr int SB = WB + AB + (A0 ? 0 : 4 * GM_TOK);  // + the rows' Q8_K d
+    static constexpr int RAW = GM_TOK * 8 * Q8_0_BYTES;         // A0: a raw buffer
+    static constexpr int AL = GM_TOK * 256 + 8 * GM_TOK * 2;    // A0: an aligned buffer: values, then fp16 d [block][token]
+    static constexpr int D = A0 ? 2 : 4 * SB <= LDS_STAGES ? 4 : 3 * SB <= LDS_STAGES ? 3 : 2;   // stages
+    static constexpr int SMEM = D * SB + (A0 ? 2 * RAW + 2 * AL : 0);
     static constexpr int N4 = TB / 1024, NR = TB - 1024 * N4, N1 = (NR + 255) / 256;   // tile DMAs: 1 KB, then 256 B
     static constexpr int L = N4 + N1 + NA + 1;                  // DMA instructions per wave and step
+    static constexpr int XCH = WB + AB;                         // bytes of a consumed stage the epilogue's exchange takes
     static_assert(W == 8 || W == 16, "8 or 16 waves");
-    static_assert(TB % 16 == 0 && NR % 4 == 0 && SB % 16 == 0, "DMA granules");
-    static_assert(D * SB <= LDS_STAGES, "stages fit");
+    static_assert(TB % 16 == 0 && NR % 4 == 0 && SB % 16 == 0 && RAW % 16 == 0 && AL % 16 == 0, "DMA granules");
+    static_assert(SMEM <= LDS_STAGES, "stages fit");
     static_assert((D - 2) * L <= 63, "vmcnt range");
 };
 // Q4_K and IQ4_XS gate/up (whose step fits 128 registers): two blocks of 8 waves per CU, each block's stream
@@ -845,6 +860,212 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
     asm volatile("");   // keeps the tile-count variants from being merged
 }
 
+// ------------------------------------------------------------------ Q8_0 activations
+// One 256-value span of the staged rows from the raw buffer (row t at 272 t: blocks of fp16 d and 32 int8) into the
+// aligned one: block c of token t in 16-byte pieces 2 c and 2 c + 1 of row t, a piece stored at piece ^ (t % 16), the
+// block's dwords reordered so that lane quarter q's 8 values of the MFMA (4 q .. + 3 and 16 + 4 q .. + 3, the two nibbles
+// of weight bytes 4 q .. + 3) are 8 contiguous bytes; d at [c][t].  A wave takes block c = wave % 8 of 32 (8 waves: 64)
+// tokens: 16 tokens x 4 quarters a pass, the block's alignment uniform over the wave.  Raw reads end 4 bytes past the raw
+// row at most (inside LDS; those bytes are shifted out).
+template <int W> struct Relay {
+    static constexpr int N = GM_TOK / W / 2;
+    uint32_t w[N][4];
+    uint16_t d;
+    static __device__ __forceinline__ int tok0(int wave) { return W == 16 ? 32 * (wave >> 3) : 0; }
+    __device__ __forceinline__ void load(const uint8_t *raw, int wave) {
+        const int lid = lane_id_here(), c = wave & 7, t0 = tok0(wave);
+        const uint32_t sb = 2u * (uint32_t) (~c & 1);   // 34 c + 2 is 2 mod 4 for even c
+        const uint8_t *p = raw + (t0 + (lid >> 2)) * 272 + 34 * c + 2 + 4 * (lid & 3) - sb;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint32_t *v = (const uint32_t *) (p + 16 * 272 * i);
+            w[i][0] = v[0]; w[i][1] = v[1]; w[i][2] = v[4]; w[i][3] = v[5];
+        }
+        d = ld_u16(raw + (t0 + (W == 16 ? lid & 31 : lid)) * 272 + 34 * c);
+    }
+    __device__ __forceinline__ void store(uint8_t *al, int wave) const {
+        const int lid = lane_id_here(), q = lid & 3, c = wave & 7, t0 = tok0(wave), t = t0 + (lid >> 2);
+        const uint32_t sb = 2u * (uint32_t) (~c & 1);
+        uint8_t *p = al + t * 256 + 16 * ((2 * c + (q >> 1)) ^ (t & 15)) + 8 * (q & 1);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            *(uint2 *) (p + 16 * 256 * i) = make_uint2(__builtin_amdgcn_alignbyte(w[i][1], w[i][0], sb), __builtin_amdgcn_alignbyte(w[i][3], w[i][2], sb));
+        *(uint16_t *) (al + GM_TOK * 256 + 2 * (GM_TOK * c + t0 + (W == 16 ? lid & 31 : lid))) = d;
+    }
+};
+
+// A weight row's span (in LDS) as lane quarter q needs it: per block c the B words of values 4 q .. + 3 and 16 + 4 q ..,
+// and the block's scale.  Block offsets are compile-time, so every read is a dword at its natural alignment (two joined
+// where the block's quants are not).  magic: the fold's product d D may be taken as fma(D + 1.5 2^23, d, -1.5 2^23 d) (see
+// step_a0), which needs d with at most 12 significant bits (fp16).
+template <int T> struct A0Row;
+__device__ __forceinline__ uint32_t ld4_off(const uint8_t *p, int off) {   // off & 3: compile-time after unrolling
+    const uint32_t *w = (const uint32_t *) (p - (off & 3));
+    return (off & 3) ? __builtin_amdgcn_alignbyte(w[1], w[0], (uint32_t) (off & 3)) : w[0];
+}
+template <> struct A0Row<IQ4_NL> {
+    static constexpr bool magic = true;
+    uint32_t w[8];
+    __device__ __forceinline__ void load(const uint8_t *row, int q, float (&d)[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) { w[c] = ld4_off(row + 18 * c + 2 + 4 * q, 18 * c + 2); d[c] = h2f(ld_u16(row + 18 * c)); }
+    }
+    __device__ __forceinline__ long b(int c, int) const { return mk_long(kv4(w[c] & 0x0F0F0F0Fu), kv4((w[c] >> 4) & 0x0F0F0F0Fu)); }
+};
+template <> struct A0Row<MXFP4> {
+    static constexpr bool magic = false;   // d up to 2^127
+    uint32_t w[8];
+    __device__ __forceinline__ void load(const uint8_t *row, int q, float (&d)[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) { w[c] = ld4_off(row + 17 * c + 1 + 4 * q, 17 * c + 1); d[c] = e8m0_half(row[17 * c]); }
+    }
+    __device__ __forceinline__ long b(int c, int) const { return mk_long(kvfp4(w[c] & 0x0F0F0F0Fu), kvfp4((w[c] >> 4) & 0x0F0F0F0Fu)); }
+};
+template <> struct A0Row<Q8_0> {
+    static constexpr bool magic = true;
+    uint32_t lo[8], hi[8];
+    __device__ __forceinline__ void load(const uint8_t *row, int q, float (&d)[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            lo[c] = ld4_off(row + 34 * c + 2 + 4 * q, 34 * c + 2);
+            hi[c] = ld4_off(row + 34 * c + 18 + 4 * q, 34 * c + 18);
+            d[c] = h2f(ld_u16(row + 34 * c));
+        }
+    }
+    __device__ __forceinline__ long b(int c, int) const { return mk_long(lo[c], hi[c]); }
+};
+template <> struct A0Row<Q5_0> {
+    static constexpr bool magic = true;
+    uint32_t w[8], h[8];   // h: the fifth bits of values 0..15 and 16..31
+    __device__ __forceinline__ void load(const uint8_t *row, int q, float (&d)[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            w[c] = ld4_off(row + 22 * c + 6 + 4 * q, 22 * c + 6);
+            h[c] = (uint32_t) ld_u16(row + 22 * c + 2) | ((uint32_t) ld_u16(row + 22 * c + 4) << 16);
+            d[c] = h2f(ld_u16(row + 22 * c));
+        }
+    }
+    __device__ __forceinline__ long b(int c, int q) const {
+        const uint32_t nh = ~h[c] >> (4 * q);
+        return mk_long((w[c] & 0x0F0F0F0Fu) | fill_f0(nh & 15), ((w[c] >> 4) & 0x0F0F0F0Fu) | fill_f0((nh >> 16) & 15));
+    }
+};
+template <> struct A0Row<Q5_1> {
+    static constexpr bool magic = false;
+    uint32_t w[8], h[8], dm[8];
+    __device__ __forceinline__ void load(const uint8_t *row, int q, float (&d)[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            w[c] = *(const uint32_t *) (row + 24 * c + 8 + 4 * q);
+            h[c] = *(const uint32_t *) (row + 24 * c + 4);
+            dm[c] = *(const uint32_t *) (row + 24 * c);
+            d[c] = h2f(dm[c] & 0xffff);
+        }
+    }
+    __device__ __forceinline__ long b(int c, int q) const {
+        const uint32_t hh = h[c] >> (4 * q);
+        return mk_long((w[c] & 0x0F0F0F0Fu) | (spread4(hh & 15) << 4), ((w[c] >> 4) & 0x0F0F0F0Fu) | (spread4((hh >> 16) & 15) << 4));
+    }
+};
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+
+// One span's step for 16 weight rows and NT token tiles: per block c one 16x16x32 MFMA a tile, folded at once, acc =
+// fma(x_d, t, acc) with t = d D (Q5_1: fma(d, D, m S), S the token block's sum from an MFMA against ones).  MAGIC: the
+// MFMA starts from 0x4B400000, so its result read as a float is D + 1.5 2^23 exactly (|D| < 2^22), and t = fma(that, d,
+// -1.5 2^23 d) is d D rounded once -- 1.5 2^23 d is exact for a finite fp16 d -- in one operation where a conversion and
+// a product take two: the fold is what bounds these types (VALU).
+template <int T, int NT, bool FIRST, bool MAGIC>
+__device__ __forceinline__ void step_a0(const A0Row<T> &w, const float (&d)[8], const uint8_t *al, float (&acc)[GM_TILES][4]) {
+#pragma unroll
+    for (int t = NT; t < GM_TILES; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
+    const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
+    const uint8_t *arow = al + rr * 256 + 8 * (q & 1);
+    const uint8_t *yrow = al + GM_TOK * 256 + 8 * q;
+    constexpr int M = MAGIC ? 0x4B400000 : 0;
+    const v4i z = {M, M, M, M};
+    // the MFMAs of block c + 1 go out before block c is folded (with one or two tiles: more cover their latency themselves)
+    constexpr int AHEAD = NT <= 2 ? 1 : 0;
+    v4i D[1 + AHEAD][NT], S[1 + AHEAD][NT];
+    v4h y[1 + AHEAD][NT];
+    auto mul = [&](int c) {
+        const int s = AHEAD ? c & 1 : 0, po = 16 * ((2 * c + (q >> 1)) ^ rr);
+        long A[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) A[t] = *(const long *) (arow + t * 16 * 256 + po);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) y[s][t] = *(const v4h *) (yrow + 2 * (GM_TOK * c + 16 * t));
+        const long B = w.b(c, q);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            D[s][t] = mfma16(A[t], B, z);
+            if constexpr (ysum_type(T)) S[s][t] = mfma16(A[t], mk_long(0x01010101u, 0x01010101u), z);
+        }
+    };
+    auto fold = [&](int c) {
+        const int s = AHEAD ? c & 1 : 0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                float x;
+                if constexpr (ysum_type(T)) x = __builtin_fmaf(d[c], (float) D[s][t][v], h2f(w.dm[c] >> 16) * (float) S[s][t][v]);
+                else if constexpr (MAGIC) x = __builtin_fmaf(__int_as_float(D[s][t][v]), d[c], -12582912.0f * d[c]);
+                else x = d[c] * (float) D[s][t][v];
+                acc[t][v] = __builtin_fmaf((float) y[s][t][v], x, FIRST && c == 0 ? 0.0f : acc[t][v]);
+            }
+        }
+    };
+    if constexpr (AHEAD) mul(0);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        if constexpr (AHEAD) { if (c < 7) mul(c + 1); } else mul(c);
+        fold(c);
+        asm volatile("");   // a scheduling-region boundary per block (register pressure)
+    }
+}
+// The step of wave's tile `wt` for ntile token tiles.  MAGIC needs finite scales: a span with an infinite or NaN scale in
+// any of the wave's rows (checked with 0 * d, NaN exactly then) takes the plain product.
+template <int T>
+__device__ __forceinline__ void span_a0(const uint8_t *wt, const uint8_t *al, int ntile, bool first, float (&acc)[GM_TILES][4]) {
+    const int lid = lane_id_here();
+    A0Row<T> w;
+    float d[8];
+    w.load(wt + (lid & 15) * span_bytes(T), lid >> 4, d);
+    constexpr bool M = A0Row<T>::magic;
+    if constexpr (M) {
+        float chk = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) chk = __builtin_fmaf(d[c], 0.0f, chk);
+        if (__builtin_expect(__ballot(chk != 0.0f) != 0, 0)) {
+            if (first) {
+#pragma unroll
+                for (int t = 0; t < GM_TILES; ++t)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[t][v] = 0.0f;
+            }
+            step_a0<T, GM_TILES, false, false>(w, d, al, acc);
+            return;
+        }
+    }
+    if (first) {
+        switch (ntile) {
+        case 1: step_a0<T, 1, true, M>(w, d, al, acc); break;
+        case 2: step_a0<T, 2, true, M>(w, d, al, acc); break;
+        case 3: step_a0<T, 3, true, M>(w, d, al, acc); break;
+        default: step_a0<T, 4, true, M>(w, d, al, acc); break;
+        }
+    } else {
+        switch (ntile) {
+        case 1: step_a0<T, 1, false, M>(w, d, al, acc); break;
+        case 2: step_a0<T, 2, false, M>(w, d, al, acc); break;
+        case 3: step_a0<T, 3, false, M>(w, d, al, acc); break;
+        default: step_a0<T, 4, false, M>(w, d, al, acc); break;
+        }
+    }
+}
+
 __host__ __device__ constexpr int xcd_gcd8(int n) { return (n & 7) == 0 ? 8 : (n & 3) == 0 ? 4 : (n & 1) == 0 ? 2 : 1; }
 
 
@@ -857,10 +1078,11 @@ template <int T, bool GU, int W, int B>
 __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const uint8_t *__restrict__ aq, uint64_t a_mul, const int *__restrict__ order,
                                                         const int *__restrict__ order_n, const int *__restrict__ egrp, const float *__restrict__ wts,
                                                         float *__restrict__ out) {
-    static_assert(vec_dot_type(T) != Q8_0, "the Q8_0-activation types run k_gemm_nl");
     using C = G5<T, W, B>;
-    constexpr int D = C::D, AQ = Q8K_BYTES;
-    __shared__ __align__(16) uint8_t smem[D * C::SB];   // stage s at s * SB: weights [wave][TB], activations [64][256], d [64]
+    constexpr bool A0 = C::A0;
+    constexpr int D = C::D, AQ = C::AROW;
+    // stage s at s * SB: weights [wave][TB], activations [64][256], d [64]; A0: weights only, then the raw and aligned buffers
+    __shared__ __align__(16) uint8_t smem[C::SMEM];
     __shared__ uint64_t s_scan[1024 + C::WAVES];                // per expert group: exclusive prefix of its items per tile class
     __shared__ int s_item[C::ITEMS][3];                  // first pair in order, tokens, weight slot
     __shared__ int s_pair[C::ITEMS][GM_TOK];             // pair index of each token of the segment's items
@@ -902,7 +1124,10 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     }
     uint64_t tot = 0;
     for (int w = 0; w < C::WAVES; ++w) tot += s_scan[1024 + w];
-    const int n4 = (int) (tot & 0xffff), n3 = (int) ((tot >> 16) & 0xffff), n2 = (int) ((tot >> 32) & 0xffff), n1 = (int) (tot >> 48);
+    // (scalar registers: every loop below runs on counts derived from these, and the compiler cannot see that values
+    // read from LDS are uniform)
+    const uint32_t tlo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) tot), thi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (tot >> 32));
+    const int n4 = (int) (tlo & 0xffff), n3 = (int) (tlo >> 16), n2 = (int) (thi & 0xffff), n1 = (int) (thi >> 16);
     const int total = n4 + n3 + n2 + n1;
     // Block (x, y) runs on XCD (x + gridDim.x y) % 8, and each XCD has its own L2.  This block's logical row block
     // bx and item slot y0: with gridDim.y a multiple of 8 (the host's choice from 8 slots up), XCD c takes the slots
@@ -934,6 +1159,8 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     auto stage_w = [&](int s) { return smem + s * C::SB; };
     auto stage_a = [&](int s) { return (int8_t *) (smem + s * C::SB + C::WB); };
     auto stage_d = [&](int s) { return (const float *) (smem + s * C::SB + C::WB + C::AB); };
+    auto raw_a = [&](int s) { return smem + D * C::SB + (s & 1) * C::RAW; };
+    auto al_a = [&](int s) { return smem + D * C::SB + 2 * C::RAW + (s & 1) * C::AL; };
 
     for (int seg = 0; seg < my_items; seg += C::ITEMS) {
         const int nit = min(C::ITEMS, my_items - seg);
@@ -965,68 +1192,83 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
         __syncthreads();
         const int nsteps = nit * nsb;
 
-        // ---- issue: the DMAs of step (iss_it, iss_b) into stage iss_stage, then advance (staying on the last step
-        // once there).  Activation rows: this wave's tokens 8 wave + 4 i + lane / 16 (lane l fetches 16-byte piece
-        // (l % 16) ^ (t % 16) of token t, the conflict-free layout the MFMA reads use) and, on lanes 0-7, the d of
-        // tokens 8 wave + lane.  Absent tokens are not fetched (their LDS rows keep stale bytes, whose MFMA columns
-        // are never stored); lane 0 of an instruction fetches from the item's first row when its token is absent.
-        // Offsets are bytes from aq (the caller's activations stay below 4 GB).
-        uint32_t aoff[C::NA], doff;
-        int iss_it = 0, iss_b = 0, iss_stage = 0, iss_step = 0, iss_ntok = 0;
+        // ---- issue: the DMAs of the next step of each stream (weights; activation rows, with the weights, or for A0 one
+        // step ahead of them), then advance.  What an item fixes is read at its first span: the weight and activation
+        // addresses (scalar pointers that advance by a span) and the lanes' byte offsets from the latter, NO for lanes
+        // that sit out: absent tokens are not fetched (their LDS rows keep stale bytes, whose MFMA columns are never
+        // stored).  The caller's activations stay below 4 GB.
+        constexpr uint32_t NO = 0xFFFFFFFFu;
         const uint32_t lane16 = 16 * lane, lane4 = 4 * lane;
-        auto issue = [&]() {
-            const int it = iss_it, b = iss_b;
-            if (b == 0) {
-                const int ntok = __builtin_amdgcn_readfirstlane(s_item[it][1]);   // uniform: a scalar register
-                iss_ntok = ntok;
-                const int p0 = s_pair[it][0];
+        auto row_off = [&](int it, int t, int ntok) -> uint32_t {   // the activation row of token t of an item
+            const int pr = t < ntok ? s_pair[it][t] : s_pair[it][0];
+            return (GU ? div_by_mul((uint32_t) pr, a_mul) : (uint32_t) pr) * (uint32_t) arow;
+        };
+        int w_it = 0, w_b = 0, w_step = 0;
+        const uint8_t *w_src = nullptr;
+        auto issue_w = [&](int stage) {
+            if (w_b == 0) w_src = Wmat + (size_t) __builtin_amdgcn_readfirstlane(s_item[w_it][2]) * mbytes;
+            const uint32_t wdst = lds_addr(stage_w(stage) + wave * C::TB);
+#pragma unroll
+            for (int i = 0; i < C::N4; ++i) dma_s128(w_src + 1024 * i, lane16, wdst + 1024 * i);
+#pragma unroll
+            for (int j = 0; j < C::N1; ++j)
+                if (256 * j + 4 * lane < C::NR) dma_s32(w_src + 1024 * C::N4 + 256 * j, lane4, wdst + 1024 * C::N4 + 256 * j);
+        };
+        auto next_w = [&]() { ++w_step; w_src += C::TB; if (++w_b == nsb) { w_b = 0; ++w_it; } };
+        uint32_t aoff[C::NA], doff = NO;
+        int a_it = 0, a_b = 0;
+        const uint8_t *a_src = nullptr;
+        // this wave's tokens TPW wave + 4 i + lane / 16: lane l fetches 16-byte piece (l % 16) ^ (t % 16) of token t, the
+        // conflict-free layout the MFMA reads use, and, on the first TPW lanes, the d of token TPW wave + lane; lane 0
+        // of every instruction fetches something, so that every instruction issues (the waits count them)
+        auto issue_a = [&](int stage) {
+            if (a_b == 0) {
+                const int ntok = __builtin_amdgcn_readfirstlane(s_item[a_it][1]);
+                a_src = aq;
 #pragma unroll
                 for (int i = 0; i < C::NA; ++i) {
                     const int t = C::TPW * wave + 4 * i + (lane >> 4);
-                    const int pr = t < ntok ? s_pair[it][t] : p0;
-                    aoff[i] = (GU ? div_by_mul((uint32_t) pr, a_mul) : (uint32_t) pr) * (uint32_t) arow + 4 + 16 * ((lane & 15) ^ (t & 15));
+                    aoff[i] = t < ntok || lane == 0 ? row_off(a_it, t, ntok) + 4 + 16 * ((lane & 15) ^ (t & 15)) : NO;
                 }
-                const int td = C::TPW * wave + (lane & (C::TPW - 1));
-                const int prd = td < ntok ? s_pair[it][td] : p0;
-                doff = (GU ? div_by_mul((uint32_t) prd, a_mul) : (uint32_t) prd) * (uint32_t) arow;
+                const int td = C::TPW * wave + lane;
+                doff = lane < C::TPW && (td < ntok || lane == 0) ? row_off(a_it, td, ntok) : NO;
             }
-            const int stage = iss_stage;
-            const uint8_t *wsrc = Wmat + (size_t) __builtin_amdgcn_readfirstlane(s_item[it][2]) * mbytes + (size_t) b * C::TB;
-            const uint32_t wdst = lds_addr(stage_w(stage) + wave * C::TB);
-#pragma unroll
-            for (int i = 0; i < C::N4; ++i) dma_s128(wsrc + 1024 * i, lane16, wdst + 1024 * i);
-#pragma unroll
-            for (int j = 0; j < C::N1; ++j)
-                if (256 * j + 4 * lane < C::NR) dma_s32(wsrc + 1024 * C::N4 + 256 * j, lane4, wdst + 1024 * C::N4 + 256 * j);
-            const uint32_t bo = (uint32_t) b * AQ;
             const uint32_t adst = lds_addr(stage_a(stage) + C::TPW * wave * 256);
-            // lanes of absent tokens sit out, except lane 0, so that every instruction issues (the waits count them)
 #pragma unroll
             for (int i = 0; i < C::NA; ++i)
-                if (C::TPW * wave + 4 * i + (lane >> 4) < iss_ntok || lane == 0) dma_s128(aq, aoff[i] + bo, adst + 1024 * i);
-            if (lane < C::TPW && (C::TPW * wave + lane < iss_ntok || lane == 0)) dma_s32(aq, doff + bo, lds_addr(stage_d(stage) + C::TPW * wave));
-            if (iss_step < nsteps - 1) {
-                ++iss_step;
-                if (++iss_b == nsb) { iss_b = 0; ++iss_it; }
-            }
-            iss_stage = iss_stage == D - 1 ? 0 : iss_stage + 1;
-            // uniform counters: kept in scalar registers (the compiler cannot prove them uniform by itself)
-            iss_it = __builtin_amdgcn_readfirstlane(iss_it);
-            iss_b = __builtin_amdgcn_readfirstlane(iss_b);
-            iss_step = __builtin_amdgcn_readfirstlane(iss_step);
-            iss_stage = __builtin_amdgcn_readfirstlane(iss_stage);
+                if (aoff[i] != NO) dma_s128(a_src, aoff[i], adst + 1024 * i);
+            if (doff != NO) dma_s32(a_src, doff, lds_addr(stage_d(stage) + C::TPW * wave));
         };
+        // A0: lane l of DMA i takes 16-byte piece 64 i + l of the wave's TPW rows of 17
+        auto issue_raw = [&](int buf) {
+            if (a_b == 0) {
+                const int ntok = __builtin_amdgcn_readfirstlane(s_item[a_it][1]);
+                a_src = aq;
+#pragma unroll
+                for (int i = 0; i < C::NA; ++i) {
+                    const int pc = 64 * i + lane, t = C::TPW * wave + pc / 17;
+                    aoff[i] = pc < 17 * C::TPW && t < ntok ? row_off(a_it, t, ntok) + 16 * (pc % 17) : NO;
+                }
+            }
+            const uint32_t adst = lds_addr(raw_a(buf) + 272 * C::TPW * wave);
+#pragma unroll
+            for (int i = 0; i < C::NA; ++i)
+                if (aoff[i] != NO) dma_s128(a_src, aoff[i], adst + 1024 * i);
+        };
+        auto next_a = [&]() { a_src += AQ; if (++a_b == nsb) { a_b = 0; ++a_it; } };
 
         float acc[GM_TILES][4];
 #pragma unroll
         for (int i = 0; i < GM_TILES; ++i)
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[i][v] = 0.0f;
-        auto compute = [&](int it, int b, int stage) {
-            const int ntok = __builtin_amdgcn_readfirstlane(s_item[it][1]), ntile = (ntok + 15) >> 4;   // uniform
+        auto compute = [&](int it, int b, int stage, int ntok) {
+            const int ntile = (ntok + 15) >> 4;
             const int8_t *as = stage_a(stage);
             const float *yd = stage_d(stage);
-            if constexpr (T == Q4_K) {
+            if constexpr (A0) {
+                span_a0<T>(stage_w(stage) + wave * C::TB, al_a(stage), ntile, b == 0, acc);
+            } else if constexpr (T == Q4_K) {
                 // straight-line code per tile count
                 const uint8_t *wt = stage_w(stage) + wave * C::TB;
                 static_assert(GM_TILES == 4, "one case per tile count");
@@ -1083,7 +1325,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     }
                 }
             } else {
-            Raw<T> wr;
+            Raw<A0 ? (int) Q4_K : T> wr;   // (the A0 types never come here)
             wr.load(stage_w(stage) + wave * C::TB + rr * C::BB, q);
             int si[GM_TILES][4];
             v4i sm[GM_TILES];
@@ -1130,8 +1372,8 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             constexpr int OR = GU ? 16 * C::HALF : C::ROWS;   // output rows of the block
             constexpr int LD = OR + 1;                         // floats per token in LDS
             constexpr int NCOPY = GU ? 2 : 1;
-            constexpr int TOKP = NCOPY * 64 * LD * 4 <= C::WB + C::AB ? 64 : NCOPY * 32 * LD * 4 <= C::WB + C::AB ? 32 : 16;
-            static_assert(NCOPY * TOKP * LD * 4 <= C::WB + C::AB, "the exchange fits in a stage");
+            constexpr int TOKP = NCOPY * 64 * LD * 4 <= C::XCH ? 64 : NCOPY * 32 * LD * 4 <= C::XCH ? 32 : 16;
+            static_assert(NCOPY * TOKP * LD * 4 <= C::XCH, "the exchange fits in a stage");
             float *s_o = (float *) stage_w(stage);             // gate (or down) values
             float *s_u = s_o + TOKP * LD;                      // up values
             const int row0 = bx * OR;
@@ -1157,7 +1399,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     for (int r = lane; r < OR; r += 64) store_f32(o + r, GU ? hy_swiglu(so[r], su[r], m.clamp) : wt * so[r]);
                 }
             }
-            if constexpr (T != Q4_K && T != Q6_K && T != IQ2_XS) {   // (those types' steps start the next item's sums themselves)
+            if constexpr (!A0 && T != Q4_K && T != Q6_K && T != IQ2_XS) {   // (those types' steps start the next item's sums themselves)
 #pragma unroll
                 for (int tile = 0; tile < GM_TILES; ++tile)
 #pragma unroll
@@ -1165,16 +1407,59 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             }
         };
 
+        int ntok = __builtin_amdgcn_readfirstlane(s_item[0][1]);   // of the item in progress
+        if constexpr (A0) {
+            Relay<W> rl;
+            issue_w(0);
+            next_w();
+            issue_raw(0);
+            next_a();
+            wait_vm<0>();
+            lds_barrier();
+            if (nsteps > 1) { issue_raw(1); next_a(); }
+            rl.load(raw_a(0), wave);
+            rl.store(al_a(0), wave);
+            for (int st = 0, it = 0, b = 0; st < nsteps; ++st) {
+                wait_vm<0>();
+                lds_barrier();   // weights st, raw rows st + 1 and aligned rows st are in place; step st - 1 is done with its own
+                const bool more = st + 1 < nsteps;
+                if (more) {
+                    issue_w(st + 1 & 1);
+                    next_w();
+                    if (st + 2 < nsteps) { issue_raw(st); next_a(); }
+                    rl.load(raw_a(st + 1), wave);   // (its LDS reads land while the step's weights are decoded)
+                }
+                compute(it, b, st & 1, ntok);
+                if (more) rl.store(al_a(st + 1), wave);
+                if (++b == nsb) {
+                    b = 0;
+                    ++it;
+                    if (it < nit) ntok = __builtin_amdgcn_readfirstlane(s_item[it][1]);
+                }
+            }
+            continue;
+        }
         // the stream: steps 0 .. D - 2 issued ahead; past the end, the last step is issued again (into the stage
         // of step s - 1, which nobody reads any more) so that every wait counts the same instructions
+        int istage = 0;
+        auto issue = [&]() {
+            issue_w(istage);
+            issue_a(istage);
+            if (w_step < nsteps - 1) { next_w(); next_a(); }
+            istage = istage == D - 1 ? 0 : istage + 1;
+        };
 #pragma unroll
         for (int s = 0; s < D - 1; ++s) issue();
         for (int st = 0, it = 0, b = 0, stage = 0; st < nsteps; ++st) {
             wait_vm<(D - 2) * C::L>();
             lds_barrier();
             issue();
-            compute(it, b, stage);
-            if (++b == nsb) { b = 0; ++it; }
+            compute(it, b, stage, ntok);
+            if (++b == nsb) {
+                b = 0;
+                ++it;
+                if (it < nit) ntok = __builtin_amdgcn_readfirstlane(s_item[it][1]);
+            }
             stage = stage == D - 1 ? 0 : stage + 1;
         }
         wait_vm<0>();   // no DMA into this block's LDS may outlive the segment
@@ -1205,9 +1490,10 @@ __device__ __forceinline__ void chunk_fold(const Raw<T> &w, int c, int q, const 
     }
 }
 
-// IQ4_NL, Q8_0, MXFP4, Q5_0 and Q5_1 weights (Q8_0 activations, whose 2-byte aligned blocks the LDS DMA above cannot stage): register-staged
-// stream, one step ahead.  A block walks the work items it, it + gridDim.y, ...; the (item, block) steps form one stream in which the
-// next step's weight and activation bytes are loaded while the current step computes, across item boundaries.
+// The types with Q8_0 activations in launches beyond k_gemm's 32-bit activation offsets or 16-bit item counts: a
+// register-staged stream, one step ahead.  A block walks the work items it, it + gridDim.y, ...; the (item, block) steps
+// form one stream in which the next step's weight and activation bytes are loaded while the current step computes, across
+// item boundaries.
 template <int T, bool GU>
 __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__restrict__ aq, int a_div, const int *__restrict__ order,
                                               const int *__restrict__ order_n, const int *__restrict__ egrp, const float *__restrict__ wts,
@@ -1420,23 +1706,47 @@ static int cu_count() {
 static int item_slots(int row_tiles, int n_pairs, int max_active, int per_cu, bool xcd = false) {
     const int want = cu_count() * per_cu / row_tiles;   // every block resident at once
     const int n = std::max(1, std::min(max_items(n_pairs, max_active), want));
-    if (xcd && n >= 8) return n / 8 * 8;
+    if (xcd && n >= 8 && n / 8 * 8 * 8 > n * 7) return n / 8 * 8;   // (unless that would idle an eighth of the blocks)
     const int P = 8 / xcd_gcd8(row_tiles);
     return n >= P ? n / P * P : n;
+}
+
+// the types with Q8_0 activations
+#define HY_A0_SWITCH(T, ...)                                                                       \
+    switch (T) {                                                                                   \
+    case IQ4_NL: { constexpr int TT = IQ4_NL; __VA_ARGS__; }                                             \
+    case MXFP4: { constexpr int TT = MXFP4; __VA_ARGS__; }                                               \
+    case Q5_0: { constexpr int TT = Q5_0; __VA_ARGS__; }                                                 \
+    case Q5_1: { constexpr int TT = Q5_1; __VA_ARGS__; }                                                 \
+    default: { constexpr int TT = Q8_0; __VA_ARGS__; }                                                   \
+    }
+// their waves a block: 16 where two weight stages of 256 rows leave room for the activation buffers, else 8
+constexpr int a0_waves(int t) { return 2 * 256 * span_bytes(t) + 4 * (GM_TOK * 8 * Q8_0_BYTES) <= 150 * 1024 ? 16 : 8; }
+// k_gemm's 32-bit activation offsets and 16-bit item counts hold (larger launches take k_gemm_nl)
+static bool a0_fits(int n_pairs, int k, int in_dim, int max_active) {
+    return (size_t) n_pairs * (in_dim / 256) * (8 * Q8_0_BYTES) < 0xFFFF0000u && (uint64_t) n_pairs * (uint64_t) k < (1ull << 32) &&
+           max_items(n_pairs, max_active) < GM_MAX_ITEMS;
 }
 
 int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs, const int *order, const int *order_n, const int *egrp,
                         int max_active, float *h, hipStream_t s) {
     if (max_active <= 0 || n_pairs <= 0) return HY_OK;
-    const int rt = (m.ff + 31) / 32;
     if (vec_dot_type(m.tg) == Q8_0) {
+        if (a0_fits(n_pairs, k, m.n, max_active)) {
+            HY_A0_SWITCH(m.tg, {
+                constexpr int W = a0_waves(TT);
+                const int rb = m.ff / (8 * W);
+                dim3 grid(rb, item_slots(rb, n_pairs, max_active, 1, true));
+                hipLaunchKernelGGL((k_gemm<TT, true, W, 1>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
+                return check_launch("hy_moe_gemm_gate_up");
+            });
+        }
+        const int rt = (m.ff + 31) / 32;
         dim3 grid(rt, item_slots(rt, n_pairs, max_active, 3));
-        if (m.tg == IQ4_NL) hipLaunchKernelGGL((k_gemm_nl<IQ4_NL, true>), grid, dim3(256), 0, s, m, (const uint8_t *) xq, k, order, order_n, egrp, nullptr, h);
-        else if (m.tg == MXFP4) hipLaunchKernelGGL((k_gemm_nl<MXFP4, true>), grid, dim3(256), 0, s, m, (const uint8_t *) xq, k, order, order_n, egrp, nullptr, h);
-        else if (m.tg == Q5_0) hipLaunchKernelGGL((k_gemm_nl<Q5_0, true>), grid, dim3(256), 0, s, m, (const uint8_t *) xq, k, order, order_n, egrp, nullptr, h);
-        else if (m.tg == Q5_1) hipLaunchKernelGGL((k_gemm_nl<Q5_1, true>), grid, dim3(256), 0, s, m, (const uint8_t *) xq, k, order, order_n, egrp, nullptr, h);
-        else hipLaunchKernelGGL((k_gemm_nl<Q8_0, true>), grid, dim3(256), 0, s, m, (const uint8_t *) xq, k, order, order_n, egrp, nullptr, h);
-        return check_launch("hy_moe_gemm_gate_up");
+        HY_A0_SWITCH(m.tg, {
+            hipLaunchKernelGGL((k_gemm_nl<TT, true>), grid, dim3(256), 0, s, m, (const uint8_t *) xq, k, order, order_n, egrp, nullptr, h);
+            return check_launch("hy_moe_gemm_gate_up");
+        });
     }
     if ((size_t) n_pairs * (m.n / 256) * Q8K_BYTES >= (1ull << 32)) { set_error("hy_moe_gemm_gate_up: activations of 4 GB or more"); return HY_EBAD_SHAPE; }
     if (k <= 0 || (uint64_t) n_pairs * (uint64_t) k >= (1ull << 32)) { set_error("hy_moe_gemm_gate_up: k out of range for the pair count"); return HY_EBAD_SHAPE; }
@@ -1463,15 +1773,22 @@ int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs,
 int launch_gemm_down(const hy_moe_dev &m, const void *hq, int n_pairs, const int *order, const int *order_n, const int *egrp, int max_active,
                      const float *wts, float *y, hipStream_t s) {
     if (max_active <= 0 || n_pairs <= 0) return HY_OK;
-    const int rt = (m.n + GM_ROWS - 1) / GM_ROWS;
     if (vec_dot_type(m.td) == Q8_0) {
+        if (a0_fits(n_pairs, 1, m.ff, max_active)) {
+            HY_A0_SWITCH(m.td, {
+                constexpr int W = a0_waves(TT);
+                const int rb = m.n / (16 * W);
+                dim3 grid(rb, item_slots(rb, n_pairs, max_active, 1, true));
+                hipLaunchKernelGGL((k_gemm<TT, false, W, 1>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) hq, div_mul_of(1), order, order_n, egrp, wts, y);
+                return check_launch("hy_moe_gemm_down");
+            });
+        }
+        const int rt = (m.n + GM_ROWS - 1) / GM_ROWS;
         dim3 grid(rt, item_slots(rt, n_pairs, max_active, 3));
-        if (m.td == IQ4_NL) hipLaunchKernelGGL((k_gemm_nl<IQ4_NL, false>), grid, dim3(256), 0, s, m, (const uint8_t *) hq, 1, order, order_n, egrp, wts, y);
-        else if (m.td == MXFP4) hipLaunchKernelGGL((k_gemm_nl<MXFP4, false>), grid, dim3(256), 0, s, m, (const uint8_t *) hq, 1, order, order_n, egrp, wts, y);
-        else if (m.td == Q5_0) hipLaunchKernelGGL((k_gemm_nl<Q5_0, false>), grid, dim3(256), 0, s, m, (const uint8_t *) hq, 1, order, order_n, egrp, wts, y);
-        else if (m.td == Q5_1) hipLaunchKernelGGL((k_gemm_nl<Q5_1, false>), grid, dim3(256), 0, s, m, (const uint8_t *) hq, 1, order, order_n, egrp, wts, y);
-        else hipLaunchKernelGGL((k_gemm_nl<Q8_0, false>), grid, dim3(256), 0, s, m, (const uint8_t *) hq, 1, order, order_n, egrp, wts, y);
-        return check_launch("hy_moe_gemm_down");
+        HY_A0_SWITCH(m.td, {
+            hipLaunchKernelGGL((k_gemm_nl<TT, false>), grid, dim3(256), 0, s, m, (const uint8_t *) hq, 1, order, order_n, egrp, wts, y);
+            return check_launch("hy_moe_gemm_down");
+        });
     }
     if ((size_t) n_pairs * (m.ff / 256) * Q8K_BYTES >= (1ull << 32)) { set_error("hy_moe_gemm_down: activations of 4 GB or more"); return HY_EBAD_SHAPE; }
     if (max_items(n_pairs, max_active) >= GM_MAX_ITEMS) { set_error("hy_moe_gemm_down: %d pairs make more than %d work items", n_pairs, GM_MAX_ITEMS - 1); return HY_EBAD_SHAPE; }
