@@ -1,22 +1,18 @@
-// Prefill / speculative-verify grouped expert GEMMs on int8 MFMA (gfx950 v_mfma_i32_16x16x32_i8).
+// Prefill / speculative-verify grouped expert GEMMs on int8 MFMA (gfx950 v_mfma_i32_16x16x32_i8 / 16x16x64_i8).
 //
-// Work item = (active expert, chunk of up to 64 of its tokens, 64 weight rows); the block's 4 waves take 16
-// rows each (gate/up: 32 output rows, waves 0-1 in gate and waves 2-3 in up, SwiGLU after an LDS exchange).
-// Items are numbered expert by expert; a block finds its (expert, chunk) from egrp with a block-wide prefix
-// of the experts' chunk counts (replaces k_moe_gemm /
-// k_moe_gemm2, src/kernels4.cu:1354-1467, :1521-1631, which dequantize to fp16 and run fp16 MMA).
-// Per 256-value block b of the K dimension:
-//   A (16 tokens x 32 k): the tokens' Q8_K bytes, staged through LDS (double-buffered) for the 4 waves;
-//   B (32 k x 16 rows):   one weight row per lane group, decoded to int8 in registers chunk by chunk;
-//   D = A B per 32-value chunk, exact int32; sumi += scale * D (one 24-bit v_mad per value and chunk: |D| < 2^23,
-//   |scale| < 2^8); the mins
-//   term of Q4_K / Q5_K is a second, chained MFMA against a B that holds the chunk's min; after the 8 chunks
-//   the block's integers fold into the fp32 accumulator with the contract's formula.
-// The next block's weight bytes and activation bytes are loaded while this block computes.
-// Operand layouts (16x16x32 i8): A lane l holds token l % 16, k = 8 (l / 16) .. + 7; B lane l holds weight row
-// l % 16 with the same k; D lane l holds row l % 16 for tokens 4 (l / 16) + v, v = 0..3.
-// Types with 16-value scale groups (Q6_K, IQ2_XS) run each chunk as two MFMAs with B zeroed in the lanes of
-// the other group (lanes 0-31 hold k 0..15, lanes 32-63 k 16..31).
+// Work item = (active expert, chunk of up to 64 of its tokens); k_gemm's blocks of 8 or 16 waves walk the items of their
+// slot, a wave owning 16 weight rows (gate/up: half of the waves in gate, half in up, SwiGLU after an LDS exchange).
+// Replaces k_moe_gemm / k_moe_gemm2, src/kernels4.cu:1354-1467, :1521-1631, which dequantize to fp16 and run fp16 MMA.
+// Per 256-value span of the K dimension:
+//   A (16 tokens x 32 or 64 k): the tokens' int8 values, staged through LDS for all waves;
+//   B (k x 16 rows):            one weight row per lane of a quarter, decoded to int8 in registers from the staged tile;
+//   D = A B, exact int32: the type's scales are either carried by B (Q4_K, Q6_K, IQ2_XS, as two int8 planes) or applied to
+//   D a 32-value chunk at a time (24-bit v_mad: |D| < 2^23, |scale| < 2^8), the mins by a chained MFMA against the chunk's
+//   min; the span's integers then fold into the fp32 accumulator with the contract's formula.  Types with Q8_0
+//   activations fold every 32-value block on its own.
+// Operand layouts (16x16x32 i8): A lane l holds token l % 16, k = 8 (l / 16) .. + 7; B lane l holds weight row l % 16 with
+// the same k; D lane l holds row l % 16 for tokens 4 (l / 16) + v, v = 0..3.  The order of k inside an MFMA is free, as
+// long as A and B agree.
 #include "hy_internal.h"
 #include "hy_blocks.cuh"
 
@@ -79,22 +75,29 @@ template <> struct Raw<Q4_K> {   // 144 B: d, dmin, scales[12], qs[128]; chunk c
 };
 template <> struct Raw<Q5_K> {   // 176 B: + qh[32] @16 (bit c of qh[l] is bit 4 of chunk c's value l), qs @48
     static constexpr bool mins = true, g16 = false, per_chunk = false;
-    uint4 hd; uint2 qv[4], qh;
+    uint2 qv[4], qh; uint32_t dm, sl, sh, ml, mh;   // scales and mins of chunks 0..3 and 4..7, a byte each
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-        hd = load16_a4(blk);
+        const uint4 hd = load16_a4(blk);
+        dm = hd.x;
+        sl = hd.y & 0x3F3F3F3Fu;
+        ml = hd.z & 0x3F3F3F3Fu;
+        sh = (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u);
+        mh = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
         qh = *(const uint2 *) (blk + 16 + 8 * q);
 #pragma unroll
         for (int jp = 0; jp < 4; ++jp) qv[jp] = *(const uint2 *) (blk + 48 + 32 * jp + 8 * q);
     }
+    static __device__ __forceinline__ uint32_t bit4(uint32_t h, int c) { return c <= 4 ? h << (4 - c) : h >> (c - 4); }   // bit c to bit 4 (of every byte, after the mask)
     __device__ __forceinline__ void chunk(int c, int, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int sh = 4 * (c & 1);
-        b0 = ((qv[c >> 1].x >> sh) & 0x0F0F0F0Fu) | (((qh.x >> c) & 0x01010101u) << 4);
-        b1 = ((qv[c >> 1].y >> sh) & 0x0F0F0F0Fu) | (((qh.y >> c) & 0x01010101u) << 4);
-        scale_min_k4(hd.y, hd.z, hd.w, c, s0, mn);
+        const int n = 4 * (c & 1);
+        b0 = (bit4(qh.x, c) & 0x10101010u) | ((qv[c >> 1].x >> n) & 0x0F0F0F0Fu);
+        b1 = (bit4(qh.y, c) & 0x10101010u) | ((qv[c >> 1].y >> n) & 0x0F0F0F0Fu);
+        s0 = (int) (((c < 4 ? sl : sh) >> (8 * (c & 3))) & 255);
+        mn = (int) (((c < 4 ? ml : mh) >> (8 * (c & 3))) & 255);
         s1 = 0;
     }
     __device__ __forceinline__ float fold(int si, int sm) const {
-        return __builtin_fmaf(h2f(hd.x & 0xffff), (float) si, -(h2f(hd.x >> 16) * (float) sm));
+        return __builtin_fmaf(h2f(dm & 0xffff), (float) si, -(h2f(dm >> 16) * (float) sm));
     }
 };
 // Q2_K (84 B: scales[16], qs[64] @16, d @80, dmin @82): chunk c = values 32 c ..: 2-bit fields 2 (c & 3) of qs bytes
@@ -496,68 +499,11 @@ template <> struct Raw<Q5_0> {
 
 constexpr int GM_TOK = 64, GM_TILES = GM_TOK / 16, GM_ROWS = 64, GM_LD = 264;   // LDS row stride of staged activations
 
-// one chunk's integers for the tiles: si[tile][v] += scale * D; sm[tile] chained for the mins
-// A-operand bytes of token row t (tile * 16 + rr), k = 32 c + 8 q .. + 7: padded rows (GM_LD bytes), or rows of 256
-// bytes whose 16-byte pieces are stored at piece ^ (t % 16) (the LDS-DMA layout; conflict-free MFMA operand reads)
-template <bool SWZ>
-__device__ __forceinline__ long a_frag(const int8_t *As, int tile, int rr, int c, int q) {
-    if constexpr (SWZ) return *(const long *) (As + (tile * 16 + rr) * 256 + 16 * ((2 * c + (q >> 1)) ^ rr) + 8 * (q & 1));
-    else return *(const long *) (As + (tile * 16 + rr) * GM_LD + 32 * c + 8 * q);
-}
-
-// (NT: a compile-time bound on the tiles; ntile, the run-time count, is NT itself where the caller specializes)
-template <int T, bool SWZ = false, int NT = GM_TILES>
-__device__ __forceinline__ void chunk_ints(const Raw<T> &w, int c, int q, const uint2 *grid, const int8_t *As, int rr, int ntile,
-                                           int (&si)[GM_TILES][4], v4i (&sm)[GM_TILES], const long (*af)[8] = nullptr) {
-    const v4i z = {0, 0, 0, 0};
-    uint32_t b0, b1;
-    int s0, s1, mn;
-    w.chunk(c, q, grid, b0, b1, s0, s1, mn);
-    const uint32_t mb = __builtin_amdgcn_perm(0u, (uint32_t) mn, 0u);   // the min in all four bytes (selector 0-3: bytes of the 2nd operand)
-#pragma unroll
-    for (int tile = 0; tile < NT; ++tile) {
-        if (tile >= ntile) break;
-        const long a = af ? af[tile][c] : a_frag<SWZ>(As, tile, rr, c, q);   // af: read up front by the caller
-        if constexpr (Raw<T>::g16) {
-            const bool lo = q < 2;
-            const v4i d0 = mfma16(a, mk_long(lo ? b0 : 0u, lo ? b1 : 0u), z);
-            const v4i d1 = mfma16(a, mk_long(lo ? 0u : b0, lo ? 0u : b1), z);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) si[tile][v] += __mul24(s0, d0[v]) + __mul24(s1, d1[v]);
-            if constexpr (Raw<T>::mins) sm[tile] = mfma16(a, mk_long(mb, mb), sm[tile]);   // mb: the lane's group's min
-        } else {
-            const v4i d0 = mfma16(a, mk_long(b0, b1), z);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) si[tile][v] += __mul24(s0, d0[v]);
-            if constexpr (Raw<T>::mins) sm[tile] = mfma16(a, mk_long(mb, mb), sm[tile]);
-        }
-    }
-}
-
-
-// each Raw<T> register set: wait until its loads have landed (every register is an input of an empty asm)
-template <class R> __device__ __forceinline__ void touch_regs(const R &r) {
-    static_assert(sizeof(R) % 4 == 0, "register set of whole dwords");
-    const uint32_t *w = (const uint32_t *) &r;
-#pragma unroll
-    for (int i = 0; i < (int) (sizeof(R) / 4); ++i) asm volatile("" ::"v"(w[i]));
-}
-
 // Direct global -> LDS loads and the epilogue's stores, issued from inline asm so that the compiler's wait
 // bookkeeping sees only the weight loads of the stream.  (Its bookkeeping treats LDS loads, register loads and
 // stores as possibly completing out of order and would then wait for all of them at every step.)  Vector memory
 // operations of a wave complete in issue order, so waiting for a step's weight registers also covers every DMA
 // issued before them.  M0 holds the LDS address of a DMA; it is saved and restored around it.
-__device__ __forceinline__ void dma_lds_b32(const void *g, uint32_t lds) {
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
-}
-__device__ __forceinline__ void dma_lds_b128(const void *g, uint32_t lds) {
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(g), "s"(__builtin_amdgcn_readfirstlane(lds)) : "memory");
-}
 __device__ __forceinline__ void store_f32(float *g, float v) { asm volatile("global_store_dword %0, %1, off" ::"v"(g), "v"(v) : "memory"); }
 
 // ------------------------------------------------------------------ the grouped GEMM stream
@@ -607,15 +553,22 @@ template <int T, int W, int B> struct G5 {
     static constexpr int L = N4 + N1 + NA + 1;                  // DMA instructions per wave and step
     static constexpr int XCH = WB + AB;                         // bytes of a consumed stage the epilogue's exchange takes
     static_assert(W == 8 || W == 16, "8 or 16 waves");
-    static_assert(TB % 16 == 0 && NR % 4 == 0 && SB % 16 == 0 && RAW % 16 == 0 && AL % 16 == 0, "DMA granules");
+    static_assert(TB % 16 == 0 && NR % 4 == 0, "DMA granules");
+    static_assert(WB % 256 == 0 && SB % 256 == 0 && RAW % 256 == 0 && AL % 256 == 0, "activation rows at multiples of 256 (lds_at)");
     static_assert(SMEM <= LDS_STAGES, "stages fit");
     static_assert((D - 2) * L <= 63, "vmcnt range");
 };
-// Q4_K and IQ4_XS gate/up (whose step fits 128 registers): two blocks of 8 waves per CU, each block's stream
-// running independently of the other's; the rest: one block of 8 waves (up to 256 registers, deeper rings)
-template <int T, bool GU> constexpr int g5_blocks() { return GU && (T == Q4_K || T == IQ4_XS) ? 2 : 1; }
+// Q4_K gate/up (whose step fits 128 registers): two blocks of 8 waves per CU, each block's stream running independently
+// of the other's; wide_type: one block of 16 waves (256 weight rows share every activation read; the step fits 128
+// registers); the rest: one block of 8 waves (up to 256 registers, deeper rings)
+template <int T, bool GU> constexpr int g5_blocks() { return GU && T == Q4_K ? 2 : 1; }
+constexpr bool wide_type(int t) { return t == IQ2_XS || t == IQ4_XS; }
 
 __device__ __forceinline__ v4i mfma64(v4i a, v4i b, v4i c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
+// Operand reads of the activation rows.  Row t (256 bytes, at a multiple of 256) holds its 16-byte pieces at piece ^ (t %
+// 16), so the piece p ^ k of a lane's row, p its first one and k compile-time, sits at the first one's address ^ 16 k: one
+// operation a read where piece, row and stage take three.
+template <typename V> __device__ __forceinline__ V lds_at(uint32_t addr) { return *(const __attribute__((address_space(3))) V *) (uintptr_t) addr; }
 typedef unsigned short v2u16 __attribute__((ext_vector_type(2)));
 // byte `b` of x in both 16-bit halves / in all four bytes
 __device__ __forceinline__ uint32_t bcast16(uint32_t x, int b) { return __builtin_amdgcn_perm(0u, x, 0x0C000C00u | (uint32_t) b | ((uint32_t) b << 16)); }
@@ -657,7 +610,7 @@ __device__ __forceinline__ void step_q4k(const uint8_t *wl0, const int8_t *as, c
     const uint32_t m_hi = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
     const int hs = q >> 1;                   // 1: this lane takes the odd chunk of each pair (the high nibbles)
     const uint32_t nsh = 4u * (uint32_t) hs;
-    const int8_t *arow = as + rr * 256;      // token row rr of tile 0; piece p of row t sits at p ^ (t % 16)
+    const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * (q ^ rr);   // token row rr of tile 0, piece q
     const v4i z = {0, 0, 0, 0};
     v4i d1[NT], d2[NT], dm[NT];
 #pragma unroll
@@ -672,10 +625,10 @@ __device__ __forceinline__ void step_q4k(const uint8_t *wl0, const int8_t *as, c
         const v4i B2 = {mul_bytes(n0, b), mul_bytes(n1, b), mul_bytes(n2, b), mul_bytes(n3, b)};
         const int mm = (int) bcast8(mp, c);
         const v4i Bm = {mm, mm, mm, mm};
-        const int po = 16 * ((4 * j + q) ^ rr);
+        const uint32_t aj = a0 ^ (64 * j);   // piece 4 j + q
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const v4i A = *(const v4i *) (arow + (T0 + t) * 16 * 256 + po);
+            const v4i A = lds_at<v4i>(aj + (T0 + t) * 16 * 256);
             d1[t] = mfma64(A, B1, j ? d1[t] : z);
             d2[t] = mfma64(A, B2, j ? d2[t] : z);
             dm[t] = mfma64(A, Bm, j ? dm[t] : z);
@@ -722,7 +675,7 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
     const uint32_t sb = 2u * (uint32_t) (rr & 1);   // the tile starts dword-aligned; a 210-byte row shifts by 2
     const uint4 scq = ld16_u2(blk + 192, sb);       // the 16 group scales (int8)
     const float d = h2f(ld_u16(blk + 208));
-    const int8_t *arow = as + rr * 256;
+    const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * (q ^ rr);   // token row rr of tile 0, piece q
     const v4i z = {0, 0, 0, 0};
     v4i dh[NT], dl[NT];
     uint4 ql, qh;
@@ -753,10 +706,10 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
             H[i] = (int) __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, ho), __builtin_bit_cast(uint32_t, he), 0x06040200u);
         }
         const v4i Bh = {H[0], H[1], H[2], H[3]}, Bl = {L[0], L[1], L[2], L[3]};
-        const int po = 16 * ((4 * j + q) ^ rr);
+        const uint32_t aj = a0 ^ (64 * j);   // piece 4 j + q
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const v4i A = *(const v4i *) (arow + (T0 + t) * 16 * 256 + po);
+            const v4i A = lds_at<v4i>(aj + (T0 + t) * 16 * 256);
             dh[t] = mfma64(A, Bh, j ? dh[t] : z);
             dl[t] = mfma64(A, Bl, j ? dl[t] : z);
             asm volatile("");   // a scheduling-region boundary: operands are not hoisted across tiles (register pressure)
@@ -818,7 +771,7 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
     for (int j = 0; j < 4; ++j) w[j] = ld4_u2(blk + 2 + 16 * j + 4 * q, al);
     const uint32_t sc0 = ld4_u2(blk + 66, al) >> (4 * q), sc1 = ld4_u2(blk + 70, al) >> (4 * q);   // group 4 j + q: nibble 0 / 4
     const float d = h2f(ld_u16(blk)) * 0.125f;
-    const int8_t *arow = as + rr * 256;
+    const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * (q ^ rr);   // token row rr of tile 0, piece q
     const v4i z = {0, 0, 0, 0};
     v4i dp[NT], dq[NT];
     uint32_t ga[4], sa[4], gb[4], sb[4];   // every lookup of the step goes out before the first MFMA
@@ -840,10 +793,10 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
                         (int) __builtin_amdgcn_perm(Pn, Pp, i2), (int) __builtin_amdgcn_perm(Pn, Pp, i3)};
         const v4i BQ = {(int) __builtin_amdgcn_perm(Qn, Qp, i0), (int) __builtin_amdgcn_perm(Qn, Qp, i1),
                         (int) __builtin_amdgcn_perm(Qn, Qp, i2), (int) __builtin_amdgcn_perm(Qn, Qp, i3)};
-        const int po = 16 * ((4 * j + q) ^ rr);
+        const uint32_t aj = a0 ^ (64 * j);   // piece 4 j + q
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const v4i A = *(const v4i *) (arow + (T0 + t) * 16 * 256 + po);
+            const v4i A = lds_at<v4i>(aj + (T0 + t) * 16 * 256);
             dp[t] = mfma64(A, BP, j ? dp[t] : z);
             dq[t] = mfma64(A, BQ, j ? dq[t] : z);
             asm volatile("");   // a scheduling-region boundary: operands are not hoisted across tiles (register pressure)
@@ -857,6 +810,77 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
             acc[T0 + t][v] = __builtin_fmaf(yd[(T0 + t) * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[T0 + t][v]);
         }
     }
+    asm volatile("");   // keeps the tile-count variants from being merged
+}
+
+// The step of the other types: per 32-value chunk a 16x16x32 MFMA a tile (16-value scale groups: two, each with the other
+// group's lanes of B zeroed), si += scale D with 24-bit multiply-adds, the mins chained in an MFMA against the chunk's min.
+// Straight-line code per tile count; with one or two tiles the MFMAs of chunk c + 1 go out before chunk c is scaled.  (A
+// run-time tile loop took its branches at every chunk; without the empty asm on each sum the compiler regrouped the
+// chunks' sums and spilled.)  IQ4_XS, 1000 tokens, 288 experts, d 4096, ff 1536, top-8: the layer call 1252 -> 1185 us,
+// with 16 waves a block and the lds_at addresses; bound by VALU issue (82 % of the cycles in gate/up).
+template <int T, int NT, bool FIRST>
+__device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, const int8_t *as, const float *yd, float (&acc)[GM_TILES][4]) {
+#pragma unroll
+    for (int t = NT; t < GM_TILES; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
+    constexpr bool G = Raw<T>::g16, MN = Raw<T>::mins;
+    const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
+    Raw<T> w;
+    w.load(wt + rr * span_bytes(T), q);
+    const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * ((q >> 1) ^ rr) + 8 * (q & 1);   // row rr of tile 0, chunk 0
+    const v4i z = {0, 0, 0, 0};
+    constexpr int AHEAD = NT <= 2 ? 1 : 0;
+    v4i D[1 + AHEAD][NT], E[1 + AHEAD][NT], sm[NT];
+    int s0[1 + AHEAD], s1[1 + AHEAD], si[NT][4];
+    auto mul = [&](int c) {
+        const int s = AHEAD ? c & 1 : 0;
+        const uint32_t ac = a0 ^ (32 * c);
+        long A[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) A[t] = lds_at<long>(ac + t * 16 * 256);
+        uint32_t b0, b1;
+        int mn;
+        w.chunk(c, q, grid, b0, b1, s0[s], s1[s], mn);
+        const uint32_t mb = __builtin_amdgcn_perm(0u, (uint32_t) mn, 0u);   // the min in all four bytes
+        const bool lo = q < 2;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if constexpr (G) {
+                D[s][t] = mfma16(A[t], mk_long(lo ? b0 : 0u, lo ? b1 : 0u), z);
+                E[s][t] = mfma16(A[t], mk_long(lo ? 0u : b0, lo ? 0u : b1), z);
+            } else {
+                D[s][t] = mfma16(A[t], mk_long(b0, b1), z);
+            }
+            if constexpr (MN) sm[t] = mfma16(A[t], mk_long(mb, mb), c ? sm[t] : z);
+        }
+    };
+    auto scale = [&](int c) {
+        const int s = AHEAD ? c & 1 : 0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                int x = c ? si[t][v] : 0;
+                x += __mul24(s0[s], D[s][t][v]);
+                if constexpr (G) x += __mul24(s1[s], E[s][t][v]);
+                asm volatile("" : "+v"(x));   // the chain of chunks is not regrouped (which kept every chunk's D live)
+                si[t][v] = x;
+            }
+    };
+    if constexpr (AHEAD) mul(0);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        if constexpr (AHEAD) { if (c < 7) mul(c + 1); } else mul(c);
+        scale(c);
+        asm volatile("");   // a scheduling-region boundary per chunk (register pressure)
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            acc[t][v] = __builtin_fmaf(yd[t * 16 + 4 * q + v], w.fold(si[t][v], MN ? sm[t][v] : 0), FIRST ? 0.0f : acc[t][v]);
     asm volatile("");   // keeps the tile-count variants from being merged
 }
 
@@ -981,7 +1005,7 @@ __device__ __forceinline__ void step_a0(const A0Row<T> &w, const float (&d)[8], 
 #pragma unroll
         for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
     const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
-    const uint8_t *arow = al + rr * 256 + 8 * (q & 1);
+    const uint32_t a0 = lds_addr(al) + rr * 256 + 16 * ((q >> 1) ^ rr) + 8 * (q & 1);   // row rr of tile 0, block 0
     const uint8_t *yrow = al + GM_TOK * 256 + 8 * q;
     constexpr int M = MAGIC ? 0x4B400000 : 0;
     const v4i z = {M, M, M, M};
@@ -990,10 +1014,11 @@ __device__ __forceinline__ void step_a0(const A0Row<T> &w, const float (&d)[8], 
     v4i D[1 + AHEAD][NT], S[1 + AHEAD][NT];
     v4h y[1 + AHEAD][NT];
     auto mul = [&](int c) {
-        const int s = AHEAD ? c & 1 : 0, po = 16 * ((2 * c + (q >> 1)) ^ rr);
+        const int s = AHEAD ? c & 1 : 0;
+        const uint32_t ac = a0 ^ (32 * c);
         long A[NT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) A[t] = *(const long *) (arow + t * 16 * 256 + po);
+        for (int t = 0; t < NT; ++t) A[t] = lds_at<long>(ac + t * 16 * 256);
 #pragma unroll
         for (int t = 0; t < NT; ++t) y[s][t] = *(const v4h *) (yrow + 2 * (GM_TOK * c + 16 * t));
         const long B = w.b(c, q);
@@ -1082,7 +1107,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     constexpr bool A0 = C::A0;
     constexpr int D = C::D, AQ = C::AROW;
     // stage s at s * SB: weights [wave][TB], activations [64][256], d [64]; A0: weights only, then the raw and aligned buffers
-    __shared__ __align__(16) uint8_t smem[C::SMEM];
+    __shared__ __align__(256) uint8_t smem[C::SMEM];
     __shared__ uint64_t s_scan[1024 + C::WAVES];                // per expert group: exclusive prefix of its items per tile class
     __shared__ int s_item[C::ITEMS][3];                  // first pair in order, tokens, weight slot
     __shared__ int s_pair[C::ITEMS][GM_TOK];             // pair index of each token of the segment's items
@@ -1325,44 +1350,23 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     }
                 }
             } else {
-            Raw<A0 ? (int) Q4_K : T> wr;   // (the A0 types never come here)
-            wr.load(stage_w(stage) + wave * C::TB + rr * C::BB, q);
-            int si[GM_TILES][4];
-            v4i sm[GM_TILES];
-#pragma unroll
-            for (int i = 0; i < GM_TILES; ++i) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) si[i][v] = 0;
-                sm[i] = v4i{0, 0, 0, 0};
-            }
-            if constexpr (B == 1 && W == 8) {
-                // the step's activation fragments (tile, chunk) read from LDS up front: one LDS round trip a step
-                // instead of one per chunk and tile (the register budget of one 8-wave block per CU has room for them)
-                long af[GM_TILES][8];
-#pragma unroll
-                for (int tile = 0; tile < GM_TILES; ++tile) {
-                    if (tile >= ntile) break;
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) af[tile][c] = a_frag<true>(as, tile, rr, c, q);
+                const uint8_t *wt = stage_w(stage) + wave * C::TB;
+                constexpr int TT = A0 ? (int) Q4_K : T;   // (the A0 types never come here)
+                if (b == 0) {
+                    switch (ntile) {
+                    case 1: step_gen<TT, 1, true>(wt, grid, as, yd, acc); break;
+                    case 2: step_gen<TT, 2, true>(wt, grid, as, yd, acc); break;
+                    case 3: step_gen<TT, 3, true>(wt, grid, as, yd, acc); break;
+                    default: step_gen<TT, 4, true>(wt, grid, as, yd, acc); break;
+                    }
+                } else {
+                    switch (ntile) {
+                    case 1: step_gen<TT, 1, false>(wt, grid, as, yd, acc); break;
+                    case 2: step_gen<TT, 2, false>(wt, grid, as, yd, acc); break;
+                    case 3: step_gen<TT, 3, false>(wt, grid, as, yd, acc); break;
+                    default: step_gen<TT, 4, false>(wt, grid, as, yd, acc); break;
+                    }
                 }
-#pragma unroll
-                for (int c = 0; c < 8; ++c) chunk_ints<T, true>(wr, c, q, grid, as, rr, ntile, si, sm, af);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    chunk_ints<T, true>(wr, c, q, grid, as, rr, ntile, si, sm);
-                    // 16 waves (128 registers): a scheduling-region boundary per chunk, so that the next chunks'
-                    // operand reads are not hoisted into this one (which spilled)
-                    if constexpr (W == 16) asm volatile("");
-                }
-            }
-#pragma unroll
-            for (int tile = 0; tile < GM_TILES; ++tile) {
-                if (tile >= ntile) break;
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    acc[tile][v] = __builtin_fmaf(yd[tile * 16 + 4 * q + v], wr.fold(si[tile][v], sm[tile][v]), acc[tile][v]);
-            }
             }
             if (b != nsb - 1) return;
             // ---- the item's outputs, through this stage (every wave has finished reading it after a barrier), TOKP
@@ -1398,12 +1402,6 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
 #pragma unroll
                     for (int r = lane; r < OR; r += 64) store_f32(o + r, GU ? hy_swiglu(so[r], su[r], m.clamp) : wt * so[r]);
                 }
-            }
-            if constexpr (!A0 && T != Q4_K && T != Q6_K && T != IQ2_XS) {   // (those types' steps start the next item's sums themselves)
-#pragma unroll
-                for (int tile = 0; tile < GM_TILES; ++tile)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[tile][v] = 0.0f;
             }
         };
 
@@ -1499,11 +1497,10 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
                                               const int *__restrict__ order_n, const int *__restrict__ egrp, const float *__restrict__ wts,
                                               float *__restrict__ out) {
     __shared__ __align__(16) int8_t As[2][GM_TOK * GM_LD];
-    constexpr bool NL = vec_dot_type(T) == Q8_0;     // Q8_0 activations, per-block fold (IQ4_NL, Q8_0, MXFP4, Q5_0, Q5_1)
-    __shared__ float Yd[2][GM_TOK * (NL ? 8 : 1)];
+    static_assert(vec_dot_type(T) == Q8_0, "Q8_0 activations, a fold per 32-value block");
+    __shared__ float Yd[2][GM_TOK * 8];
     __shared__ int s_scan[1024 + 8];
     __shared__ float s_up[GU ? 32 * GM_TOK : 1];
-    __shared__ uint2 grid[iq2_lds(T)];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, rr = lane & 15, q = lane >> 4;
     const int na = order_n[1];
     // ---- items: expert group g owns ceil(cnt_g / GM_TOK) of them; s_scan = exclusive prefix (block-wide)
@@ -1525,7 +1522,6 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
         int ex = base + inc - loc;
 #pragma unroll
         for (int i = 0; i < 4; ++i) { s_scan[4 * tid + i] = ex; ex += c4[i]; }
-        if constexpr (iq2_type(T)) expand_iq2_grid<T>(grid);
         __syncthreads();
     }
     const int total = s_scan[1024] + s_scan[1025] + s_scan[1026] + s_scan[1027];
@@ -1537,9 +1533,9 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
     const bool row_ok = row < rows;
     const size_t mbytes = GU ? m.gate_bytes : m.down_bytes;
     const uint8_t *Wbase = (GU ? (wave < 2 ? m.gate : m.up) : m.down) + tiled_off(row_ok ? row : rows - 1, 0, nsb, span_bytes(T));
-    constexpr int AB = NL ? 8 * Q8_0_BYTES : Q8K_BYTES;   // activation bytes per 256 values
+    constexpr int AB = 8 * Q8_0_BYTES;   // activation bytes per 256 values
     const size_t arow = (size_t) nsb * AB;
-    constexpr int BB = NL ? 8 * block_bytes(T) : block_bytes(T);   // weight bytes per 256 values
+    constexpr int BB = 8 * block_bytes(T);   // weight bytes per 256 values
     const int st_tok = tid >> 2, st_part = tid & 3;   // staging: 64 bytes of token st_tok per thread
 
     // item -> (first pair in order, tokens, weight pointer); the staging thread's activation row
@@ -1562,16 +1558,11 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
     auto load_a = [&](const uint8_t *src, int b, uint4 (&a)[4], float (&yd)[2]) {
         if (src) {
             const uint8_t *s = src + (size_t) b * AB;
-            if constexpr (NL) {   // Q8_0 blocks 2 st_part, 2 st_part + 1: qs at 68 p + 2 (2 mod 4) and 68 p + 36
-                const uint8_t *p0 = s + 2 * Q8_0_BYTES * st_part;
-                a[0] = load16_a2(p0 + 2); a[1] = load16_a2(p0 + 18);
-                a[2] = load16_a4(p0 + 36); a[3] = load16_a4(p0 + 52);
-                yd[0] = h2f(ld_u16(p0)); yd[1] = h2f(ld_u16(p0 + Q8_0_BYTES));
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = load16_a4(s + 4 + 64 * st_part + 16 * i);
-                yd[0] = *(const float *) s; yd[1] = 0.0f;
-            }
+            // Q8_0 blocks 2 st_part, 2 st_part + 1: qs at 68 p + 2 (2 mod 4) and 68 p + 36
+            const uint8_t *p0 = s + 2 * Q8_0_BYTES * st_part;
+            a[0] = load16_a2(p0 + 2); a[1] = load16_a2(p0 + 18);
+            a[2] = load16_a4(p0 + 36); a[3] = load16_a4(p0 + 52);
+            yd[0] = h2f(ld_u16(p0)); yd[1] = h2f(ld_u16(p0 + Q8_0_BYTES));
         } else {
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = make_uint4(0, 0, 0, 0);
@@ -1596,8 +1587,7 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
             uint4 *dst = (uint4 *) (As[buf] + st_tok * GM_LD + 64 * st_part);
 #pragma unroll
             for (int i = 0; i < 4; ++i) dst[i] = a[i];
-            if constexpr (NL) { Yd[buf][st_tok * 8 + 2 * st_part] = yd[0]; Yd[buf][st_tok * 8 + 2 * st_part + 1] = yd[1]; }
-            else if (st_part == 0) Yd[buf][st_tok] = yd[0];
+            Yd[buf][st_tok * 8 + 2 * st_part] = yd[0]; Yd[buf][st_tok * 8 + 2 * st_part + 1] = yd[1];
         }
         // the next step: block b + 1 of this item, or block 0 of the next item
         const bool last_b = b + 1 == nsb;
@@ -1613,28 +1603,8 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
         }
         __syncthreads();
         const int ntile = (cur.ntok + 15) / 16;
-        if constexpr (NL) {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) chunk_fold<T>(w, c, q, As[buf], Yd[buf], rr, ntile, acc);
-        } else {
-            int si[GM_TILES][4];
-            v4i sm[GM_TILES];
-#pragma unroll
-            for (int i = 0; i < GM_TILES; ++i) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) si[i][v] = 0;
-                sm[i] = v4i{0, 0, 0, 0};
-            }
-#pragma unroll
-            for (int c = 0; c < 8; ++c) chunk_ints<T>(w, c, q, grid, As[buf], rr, ntile, si, sm);
-#pragma unroll
-            for (int tile = 0; tile < GM_TILES; ++tile) {
-                if (tile >= ntile) break;
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    acc[tile][v] = __builtin_fmaf(Yd[buf][tile * 16 + 4 * q + v], w.fold(si[tile][v], sm[tile][v]), acc[tile][v]);
-            }
-        }
+        for (int c = 0; c < 8; ++c) chunk_fold<T>(w, c, q, As[buf], Yd[buf], rr, ntile, acc);
         if (last_b) {   // the item's outputs
             if (GU && wave >= 2) {
 #pragma unroll
@@ -1763,7 +1733,7 @@ int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs,
         return check_launch("hy_moe_gemm_gate_up");
     }
     HY_GEMM_SWITCH(m.tg, {
-        constexpr int W = TT == IQ2_XS ? 16 : 8, B = g5_blocks<TT, true>();
+        constexpr int W = wide_type(TT) ? 16 : 8, B = g5_blocks<TT, true>();
         const int rb = m.ff / (8 * W);   // 8 W output rows a block
         dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, B == 1));   // two blocks a CU: every slot counts
         hipLaunchKernelGGL((k_gemm<TT, true, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
@@ -1793,7 +1763,7 @@ int launch_gemm_down(const hy_moe_dev &m, const void *hq, int n_pairs, const int
     if ((size_t) n_pairs * (m.ff / 256) * Q8K_BYTES >= (1ull << 32)) { set_error("hy_moe_gemm_down: activations of 4 GB or more"); return HY_EBAD_SHAPE; }
     if (max_items(n_pairs, max_active) >= GM_MAX_ITEMS) { set_error("hy_moe_gemm_down: %d pairs make more than %d work items", n_pairs, GM_MAX_ITEMS - 1); return HY_EBAD_SHAPE; }
     HY_GEMM_SWITCH(m.td, {
-        constexpr int W = TT == Q6_K || TT == IQ2_XS ? 16 : 8, B = g5_blocks<TT, false>();   // 16 waves where the step fits 128 registers
+        constexpr int W = wide_type(TT) || TT == Q6_K ? 16 : 8, B = g5_blocks<TT, false>();
         const int rb = m.n / (16 * W);   // 16 W output rows a block
         dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, true));
         hipLaunchKernelGGL((k_gemm<TT, false, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) hq, div_mul_of(1), order, order_n, egrp, wts, y);
