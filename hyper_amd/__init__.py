@@ -93,6 +93,7 @@ SIGNATURES = {
     "hy_moe_router_q8_bf16w": (_I, [_P, _I, _I, _P, _I, _P, _I, _P, _I, _I, _P, _I, _P]),
     "hy_moe_route_gate_up": (_I, [_DEV, _P, _I, _I, _I, _P, _P, _P, _P, _P, _I, _P]),
     "hy_moe_route_gate_up_q8": (_I, [_DEV, _P, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P]),
+    "hy_moe_gate_up_q8": (_I, [_DEV, _P, _P, _I, _I, _P, _P, _I, _P]),
     "hy_moe_shared_gate_up": (_I, [_DEV, _P, _P, _I, _P]),
     "hy_moe_shared_down": (_I, [_DEV, _P, _P, _I, _P]),
     "hy_moe_down_reduce_q8": (_I, [_DEV, _P, _P, _P, _I, _P, _P, _P, _I, _I, _P]),

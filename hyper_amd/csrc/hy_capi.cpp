@@ -389,6 +389,16 @@ int hy_moe_route_gate_up_q8(const hy_moe_dev *m, const float *logits, int ls, in
     return launch_route_gate_up(*m, logits, ls, n_expert, k, xq, ids, wts, sg, h, nt, s, (uint8_t *) hq);
 }
 
+int hy_moe_gate_up_q8(const hy_moe_dev *m, const void *xq, const int32_t *ids, int n_expert, int k, float *h, void *hq, int nt,
+                      hipStream_t s) {
+    int rc = check_dev(m, "hy_moe_gate_up_q8", true, false);
+    if (rc) return rc;
+    if (!xq || !ids || !h || k <= 0 || nt < 0) { set_error("hy_moe_gate_up_q8: bad argument"); return HY_EINVAL; }
+    if (n_expert <= 0 || n_expert > m->n_expert) { set_error("hy_moe_gate_up_q8: n_expert %d out of range", n_expert); return HY_EBAD_SHAPE; }
+    if ((uintptr_t) xq & 3) { set_error("hy_moe_gate_up_q8: xq must be 4-byte aligned"); return HY_EBAD_SHAPE; }
+    return launch_gate_up_ids(*m, xq, ids, n_expert, k, h, nt, s, (uint8_t *) hq);
+}
+
 int hy_moe_down_reduce_q8(const hy_moe_dev *m, const void *hq, const int32_t *ids, const float *wts, int k, const float *shexp,
                           const float *sg, float *out, int residual, int nt, hipStream_t s) {
     int rc = check_dev(m, "hy_moe_down_reduce_q8", false, true);

@@ -864,6 +864,42 @@ int launch_route_gate_up(const hy_moe_dev &m, const float *logits, int ls, int n
 #undef HY_RGU
 }
 
+// Decode gate/up of pairs routed beforehand (ids), from the Q8 rows: the kernel route_gate_up launches after routing
+// once.  hq: also the Q8_0 hidden rows.  HY_EUNSUPPORTED_TYPE beyond the kernel's row or slot-table limits.
+int launch_gate_up_ids(const hy_moe_dev &m, const void *xq, const int *ids, int ne, int k, float *h, int nt, hipStream_t s, uint8_t *hq) {
+    const int ng = m.n / 256, nb = m.n / block_elems(m.tg);
+    if (2 * ng > 8 * DEC_MAXP || 2 * nb > DEC_GU_TV || ne > 1024 || m.gate_bytes >= ((size_t) 1 << 32) || (long) nt * k > 65535) {
+        set_error("hy_moe_gate_up_q8: n = %d, %d experts of %zu bytes, %d pairs exceed the kernel's limits", m.n, ne, m.gate_bytes, nt * k);
+        return HY_EUNSUPPORTED_TYPE;
+    }
+    if (hq && (vec_dot_type(m.tg) != Q8_0 || vec_dot_type(m.td) != Q8_0 || 4 * 2 * nb > 2 * DEC_GU_TV)) {
+        set_error("hy_moe_gate_up_q8: Q8_0 hidden rows need gate/up and down types with Q8_0 rows and n <= 4096 (types %d/%d, n %d)", m.tg, m.td, m.n);
+        return HY_EUNSUPPORTED_TYPE;
+    }
+    if (nt == 0) return HY_OK;
+    int *idw = const_cast<int *>(ids);   // read only for pairs routed beforehand
+    if (hq) {
+        dim3 grid(m.ff / 32, nt * k);
+#define HY_GUQ(TQ) hipLaunchKernelGGL((k_route_gate_up<TQ, -16, DEC_PIPE_NP, true, true>), grid, dim3(64 * DEC_GU_WAVES), 0, s, m, nullptr, 0, ne, k, (const uint8_t *) xq, idw, nullptr, nullptr, h, 4, 2, 0, hq)
+        if (m.tg == IQ4_NL) { HY_GUQ(IQ4_NL); } else if (m.tg == MXFP4) { HY_GUQ(MXFP4); } else if (m.tg == Q5_0) { HY_GUQ(Q5_0); }
+        else if (m.tg == Q5_1) { HY_GUQ(Q5_1); }
+        else { HY_GUQ(Q8_0); }
+#undef HY_GUQ
+        return check_launch("hy_moe_gate_up_q8");
+    }
+    int rw = 1;   // rows per wave, as in launch_route_gate_up
+    auto nblocks = [&](int r) { return (long) ((m.ff + DEC_GU_WAVES * r - 1) / (DEC_GU_WAVES * r)) * nt * k; };
+    while (rw < 8 && nblocks(rw) > DEC_GU_BLOCKS && (rw + 1) * 2 * nb <= DEC_GU_TV) ++rw;
+    dim3 grid((m.ff + DEC_GU_WAVES * rw - 1) / (DEC_GU_WAVES * rw), nt * k);
+    const int np = (rw * ng + 7) / 8, q8 = 8 / rw, r8 = 8 % rw;
+#define HY_GUI(NN, PP) hipLaunchKernelGGL((k_route_gate_up<TT, -16, NN, false, PP>), grid, dim3(64 * DEC_GU_WAVES), 0, s, m, nullptr, 0, ne, k, (const uint8_t *) xq, idw, nullptr, nullptr, h, rw, q8, r8, nullptr)
+    HY_DEC_SWITCH(m.tg, {
+        if (np <= 1) { HY_GUI(1, false); } else if (np <= 2) { HY_GUI(2, false); } else if (np <= 4) { HY_GUI(4, false); } else { HY_GUI(DEC_PIPE_NP, true); }
+        return check_launch("hy_moe_gate_up_q8");
+    });
+#undef HY_GUI
+}
+
 // the gate/up of local expert 0 for every token (a shared expert) from the Q8 rows: k_route_gate_up without routing
 int launch_fixed_gate_up(const hy_moe_dev &m, const void *xq, float *h, int nt, hipStream_t s) {
     const int ng = m.n / 256, nb = m.n / block_elems(m.tg);

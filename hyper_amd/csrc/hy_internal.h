@@ -45,6 +45,10 @@ int launch_router_q8(const uint16_t *W, int rows, int kdim, const float *x, int 
 // hq: also write the Q8_0 rows of h (down types whose partner is Q8_0); HY_EUNSUPPORTED_TYPE where that does not apply
 int launch_route_gate_up(const hy_moe_dev &m, const float *logits, int ls, int ne, int k, const void *xq, int *ids, float *wts, float *sg,
                          float *h, int nt, hipStream_t s, uint8_t *hq = nullptr);
+// decode gate/up of pairs routed beforehand, from the Q8 rows (hq: also the Q8_0 rows of h); HY_EUNSUPPORTED_TYPE beyond
+// the kernel's limits
+int launch_gate_up_ids(const hy_moe_dev &m, const void *xq, const int *ids, int ne, int k, float *h, int nt, hipStream_t s,
+                       uint8_t *hq = nullptr);
 // SwiGLU(gate, up) of the descriptor's local expert 0 for nt Q8 rows (a shared expert's decode gate/up, no routing)
 int launch_fixed_gate_up(const hy_moe_dev &m, const void *xq, float *h, int nt, hipStream_t s);
 // the same for 2..8 tokens in one pass over the weights; HY_EUNSUPPORTED_TYPE outside its limits (use the one above)

@@ -204,6 +204,11 @@ def moe_route_gate_up_q8(m: MoeDev, logits, ls, n_expert, k, xq, ids, wts, sg, h
                                         _s(stream)))
 
 
+def moe_gate_up_q8(m: MoeDev, xq, ids, n_expert, k, h, hq, nt, stream=None):
+    """moe_gate_up of routed pairs from the Q8 rows of x; with hq also the Q8_0 hidden rows of moe_route_gate_up_q8."""
+    check(lib().hy_moe_gate_up_q8(m.ref, _p(xq), _p(ids), n_expert, k, _p(h), _p(hq), nt, _s(stream)))
+
+
 def moe_down_reduce_q8(m: MoeDev, hq, ids, wts, k, shexp, sg, out, residual, nt, stream=None):
     """moe_down_reduce (or its residual form) from the Q8_0 hidden rows of moe_route_gate_up_q8."""
     check(lib().hy_moe_down_reduce_q8(m.ref, _p(hq), _p(ids), _p(wts), k, _p(shexp), _p(sg), _p(out), int(bool(residual)), nt,
@@ -267,9 +272,11 @@ class MoeLayerRunner:
         # decode hands the hidden over as Q8_0 rows where the down type's partner is Q8_0, within the kernels' limits
         # (n <= 4096; k * ff / 32 <= 512 blocks and k * ff / 32 * 34 bytes <= 32 KiB per token)
         nbh = self.ff // 32
-        self.dec_hq = (router == "softmax" and vec_dot_type(L.tg) == GType.Q8_0 and vec_dot_type(L.td) == GType.Q8_0
+        self.dec_hq = (vec_dot_type(L.tg) == GType.Q8_0 and vec_dot_type(L.td) == GType.Q8_0
                        and self.d <= 4096 and self.k * nbh <= 512
                        and self.k * nbh * 34 <= 32768 and self.E <= 1024)
+        # the routers without a fused route + gate/up: the gate/up kernel by ids from the Q8 rows of x, within its limits
+        self.dec_ids = self.d <= 8192 and self.E <= 1024 and L.gate_bytes < 1 << 32
         self._side = None   # the shared expert's second stream, made on first use
         # decode's shared expert on a second stream: None = beyond 8 rows (up to 8 rows its gate/up and down read the
         # weights once for several rows and are shortest in order, ahead of the routed kernels: the 8-row IQ2_XS
@@ -385,19 +392,25 @@ class MoeLayerRunner:
             self._shared_decode(x, nt, self._fork_side(stream))
             self._join.record(self._side)
             shexp, joined = self.sh_y, (stream if stream is not None else torch.cuda.current_stream())
-        if self.dec_hq:
-            moe_route_gate_up_q8(self.dev, self.logits, self.ls, self.E, self.k, self.xq, self.ids, self.wts, self.sg, self.h, self.hq,
+        hq = self.hq if self.dec_hq else None
+        if self.router != "softmax":   # the fused route + gate/up kernel routes by softmax: route first
+            self._route_logits(nt, stream)
+            if self.dec_ids and nt * self.k <= 65535:
+                moe_gate_up_q8(self.dev, self.xq, self.ids, self.E, self.k, self.h, hq, nt, stream)
+            else:
+                hq = None
+                moe_gate_up(self.dev, x, x.stride(0), self.ids, self.k, self.h, nt, stream)
+        elif hq is not None:
+            moe_route_gate_up_q8(self.dev, self.logits, self.ls, self.E, self.k, self.xq, self.ids, self.wts, self.sg, self.h, hq,
                                  nt, stream)
+        else:
+            moe_route_gate_up(self.dev, self.logits, self.ls, self.E, self.k, self.xq, self.ids, self.wts, self.sg, self.h, nt, stream)
+        if hq is not None:
             out = self.out if resid is None else resid
             if joined is not None:
                 joined.wait_event(self._join)
-            moe_down_reduce_q8(self.dev, self.hq, self.ids, self.wts, self.k, shexp, self.sg, out, resid is not None, nt, stream)
+            moe_down_reduce_q8(self.dev, hq, self.ids, self.wts, self.k, shexp, self.sg, out, resid is not None, nt, stream)
             return out[:nt]
-        if self.router == "softmax":
-            moe_route_gate_up(self.dev, self.logits, self.ls, self.E, self.k, self.xq, self.ids, self.wts, self.sg, self.h, nt, stream)
-        else:   # the fused route + gate/up kernel routes by softmax: route first, then the gate/up GEMV by ids
-            self._route_logits(nt, stream)
-            moe_gate_up(self.dev, x, x.stride(0), self.ids, self.k, self.h, nt, stream)
         if joined is not None:
             joined.wait_event(self._join)
         if resid is not None:

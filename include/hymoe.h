@@ -246,6 +246,13 @@ int hy_moe_shared_gate_up(const hy_moe_dev *m, const void *xq, float *h, int nt,
    gate/up and down weights and n <= 4096, else HY_EUNSUPPORTED_TYPE. */
 int hy_moe_route_gate_up_q8(const hy_moe_dev *m, const float *logits, int ls, int n_expert, int k, const void *xq, int32_t *ids,
                             float *wts, float *sg, float *h, void *hq, int nt, hipStream_t s);
+/* Decode gate/up of pairs routed beforehand, from the Q8 rows xq (partner type of the gate type, e.g. from
+   hy_moe_router_q8): h[t*k + j] as hy_moe_gate_up gives it for expert ids[t*k + j] (pairs whose expert is not local leave
+   their h rows unwritten); n_expert bounds the ids.  hq (NULL: none): also the Q8_0 hidden rows, laid out and limited as
+   hy_moe_route_gate_up_q8's.  HY_EUNSUPPORTED_TYPE for n > 8192, more than 1024 experts or 65535 pairs (use
+   hy_moe_gate_up; replaces moe_gate_up, src/kernels4.cuh:67-68, for the routers without a fused form). */
+int hy_moe_gate_up_q8(const hy_moe_dev *m, const void *xq, const int32_t *ids, int n_expert, int k, float *h, void *hq, int nt,
+                      hipStream_t s);
 /* hy_moe_down_reduce (residual == 0) or hy_moe_down_reduce_residual (residual != 0) from those Q8_0 blocks (hq
    16-byte aligned); bit-identical to them on the h the blocks came from.  HY_EUNSUPPORTED_TYPE for other down types. */
 int hy_moe_down_reduce_q8(const hy_moe_dev *m, const void *hq, const int32_t *ids, const float *wts, int k, const float *shexp,
