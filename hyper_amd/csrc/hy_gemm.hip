@@ -558,11 +558,13 @@ template <int T, int W, int B> struct G5 {
     static_assert(SMEM <= LDS_STAGES, "stages fit");
     static_assert((D - 2) * L <= 63, "vmcnt range");
 };
-// Q4_K gate/up (whose step fits 128 registers): two blocks of 8 waves per CU, each block's stream running independently
-// of the other's; wide_type: one block of 16 waves (256 weight rows share every activation read; the step fits 128
-// registers); the rest: one block of 8 waves (up to 256 registers, deeper rings)
-template <int T, bool GU> constexpr int g5_blocks() { return GU && T == Q4_K ? 2 : 1; }
-constexpr bool wide_type(int t) { return t == IQ2_XS || t == IQ4_XS; }
+// Q4_K and IQ4_XS gate/up (whose steps fit 128 registers): two blocks of 8 waves per CU, each block's stream running
+// independently of the other's; IQ2_XS, and Q6_K and IQ4_XS down: one block of 16 waves (256 weight rows share every
+// activation read; the steps fit 128 registers); the rest: one block of 8 waves (up to 256 registers, deeper rings).
+// IQ4_XS, the 1000-token layer call: 1185 us with 16 waves for both, 1125 as here, 1136 with 2 x 8 waves for both;
+// IQ2_XS: 3511 us with 16 waves, 3508 with 2 x 8.
+template <int T, bool GU> constexpr int g5_blocks() { return GU && (T == Q4_K || T == IQ4_XS) ? 2 : 1; }
+template <int T, bool GU> constexpr int g5_waves() { return T == IQ2_XS || (!GU && (T == Q6_K || T == IQ4_XS)) ? 16 : 8; }
 
 __device__ __forceinline__ v4i mfma64(v4i a, v4i b, v4i c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
 // Operand reads of the activation rows.  Row t (256 bytes, at a multiple of 256) holds its 16-byte pieces at piece ^ (t %
@@ -817,8 +819,8 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
 // group's lanes of B zeroed), si += scale D with 24-bit multiply-adds, the mins chained in an MFMA against the chunk's min.
 // Straight-line code per tile count; with one or two tiles the MFMAs of chunk c + 1 go out before chunk c is scaled.  (A
 // run-time tile loop took its branches at every chunk; without the empty asm on each sum the compiler regrouped the
-// chunks' sums and spilled.)  IQ4_XS, 1000 tokens, 288 experts, d 4096, ff 1536, top-8: the layer call 1252 -> 1185 us,
-// with 16 waves a block and the lds_at addresses; bound by VALU issue (82 % of the cycles in gate/up).
+// chunks' sums and spilled.)  IQ4_XS, 1000 tokens, 288 experts, d 4096, ff 1536, top-8: the layer call 1252 -> 1125 us,
+// with the lds_at addresses and the geometry of g5_waves; bound by VALU issue (82 % of the cycles in gate/up).
 template <int T, int NT, bool FIRST>
 __device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, const int8_t *as, const float *yd, float (&acc)[GM_TILES][4]) {
 #pragma unroll
@@ -1733,7 +1735,7 @@ int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs,
         return check_launch("hy_moe_gemm_gate_up");
     }
     HY_GEMM_SWITCH(m.tg, {
-        constexpr int W = wide_type(TT) ? 16 : 8, B = g5_blocks<TT, true>();
+        constexpr int W = g5_waves<TT, true>(), B = g5_blocks<TT, true>();
         const int rb = m.ff / (8 * W);   // 8 W output rows a block
         dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, B == 1));   // two blocks a CU: every slot counts
         hipLaunchKernelGGL((k_gemm<TT, true, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
@@ -1763,7 +1765,7 @@ int launch_gemm_down(const hy_moe_dev &m, const void *hq, int n_pairs, const int
     if ((size_t) n_pairs * (m.ff / 256) * Q8K_BYTES >= (1ull << 32)) { set_error("hy_moe_gemm_down: activations of 4 GB or more"); return HY_EBAD_SHAPE; }
     if (max_items(n_pairs, max_active) >= GM_MAX_ITEMS) { set_error("hy_moe_gemm_down: %d pairs make more than %d work items", n_pairs, GM_MAX_ITEMS - 1); return HY_EBAD_SHAPE; }
     HY_GEMM_SWITCH(m.td, {
-        constexpr int W = wide_type(TT) || TT == Q6_K ? 16 : 8, B = g5_blocks<TT, false>();
+        constexpr int W = g5_waves<TT, false>(), B = g5_blocks<TT, false>();
         const int rb = m.n / (16 * W);   // 16 W output rows a block
         dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, true));
         hipLaunchKernelGGL((k_gemm<TT, false, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) hq, div_mul_of(1), order, order_n, egrp, wts, y);
