@@ -42,14 +42,20 @@ __host__ __device__ constexpr bool ysum_type(int t) { return t == Q5_1; }
 
 __device__ __forceinline__ float h2f(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 __device__ __forceinline__ uint16_t f2h(float f) { return __half_as_ushort(__float2half_rn(f)); }
-// four router weights at p as fp32: fp32 rows as they are; bf16 rows (uint16 bit patterns, p 8-byte aligned) widened,
-// which is exact (a bf16 value is the fp32 value with the low 16 bits zero), so both give the same products and sums
-__device__ __forceinline__ float4 ld_w4(const float *p) { return *(const float4 *) p; }
-__device__ __forceinline__ float4 ld_w4(const uint16_t *p) {
-    const uint2 v = *(const uint2 *) p;
+// four router weights at p: fp32 rows as they are, bf16 rows (uint16 bit patterns, p 8-byte aligned) as loaded (ld_w4raw),
+// and as fp32 (widen), which is exact (a bf16 value is the fp32 value with the low 16 bits zero), so both give the same
+// products and sums.  Kernels with several loads in flight keep the loaded form and widen at the use: widened at the
+// load, each load was waited for before the next went out.
+template <typename WT> struct W4Raw { using T = float4; };
+template <> struct W4Raw<uint16_t> { using T = uint2; };
+__device__ __forceinline__ float4 ld_w4raw(const float *p) { return *(const float4 *) p; }
+__device__ __forceinline__ uint2 ld_w4raw(const uint16_t *p) { return *(const uint2 *) p; }
+__device__ __forceinline__ float4 widen(float4 v) { return v; }
+__device__ __forceinline__ float4 widen(uint2 v) {
     return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
                        __uint_as_float(v.y & 0xffff0000u));
 }
+template <typename WT> __device__ __forceinline__ float4 ld_w4(const WT *p) { return widen(ld_w4raw(p)); }
 
 // exp(x) of the contract: x = n ln2 + r (ln2 = 0.693359375 - 2.12194440e-4, the first part exact in
 // 9 bits), exp(r) by the Cephes expf polynomial (S. L. Moshier), 2^n applied as two exact scalings.

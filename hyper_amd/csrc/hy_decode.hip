@@ -100,20 +100,27 @@ __global__ __launch_bounds__(256) void k_router_q8(const WT *__restrict__ W, int
     const float *xt = x + (size_t) t * xs;
     float acc = 0.0f;
     for (int e0 = 0; e0 < kdim; e0 += 256 * RB) {
-        float4 w[RB], xv[RB];
+        typename W4Raw<WT>::T w[RB];
+        float4 xv[RB];
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             const int e = e0 + 256 * i + 4 * lane;
-            w[i] = e < kdim ? ld_w4(wr + e) : make_float4(0, 0, 0, 0);
-            xv[i] = e < kdim ? *(const float4 *) (xt + e) : make_float4(0, 0, 0, 0);
+            if constexpr (sizeof(WT) == 4) {
+                w[i] = e < kdim ? ld_w4raw(wr + e) : make_float4(0, 0, 0, 0);
+                xv[i] = e < kdim ? *(const float4 *) (xt + e) : make_float4(0, 0, 0, 0);
+            } else {   // bf16: past the row's end its first values, unused (under a condition each load was waited for)
+                w[i] = ld_w4raw(wr + (e < kdim ? e : 0));
+                xv[i] = *(const float4 *) (xt + (e < kdim ? e : 0));
+            }
         }
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             if (e0 + 256 * i + 4 * lane < kdim) {
-                acc = __builtin_fmaf(w[i].x, xv[i].x, acc);
-                acc = __builtin_fmaf(w[i].y, xv[i].y, acc);
-                acc = __builtin_fmaf(w[i].z, xv[i].z, acc);
-                acc = __builtin_fmaf(w[i].w, xv[i].w, acc);
+                const float4 v = widen(w[i]);
+                acc = __builtin_fmaf(v.x, xv[i].x, acc);
+                acc = __builtin_fmaf(v.y, xv[i].y, acc);
+                acc = __builtin_fmaf(v.z, xv[i].z, acc);
+                acc = __builtin_fmaf(v.w, xv[i].w, acc);
             }
         }
     }

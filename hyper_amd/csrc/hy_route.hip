@@ -32,27 +32,31 @@ __device__ __forceinline__ void gemv_tile(const WT *__restrict__ W, int rows, in
     static_assert(RW * TW <= 64, "one bias per lane");
     float bv = 0.0f;
     if (bias && lane < RW * TW && r0 + lane / TW < rows && t0 + lane % TW < nt) bv = bias[(size_t) (t0 + lane % TW) * bs + r0 + lane / TW];
-    float4 wa[RW], xa[TW], wb[RW], xb[TW];
-    auto ld = [&](int i, float4 (&wd)[RW], float4 (&xd)[TW]) {
+    using WR = typename W4Raw<WT>::T;
+    WR wa[RW], wb[RW];
+    float4 xa[TW], xb[TW];
+    auto ld = [&](int i, WR (&wd)[RW], float4 (&xd)[TW]) {
         const int e = 256 * i + 4 * lane < kdim ? 256 * i + 4 * lane : 4 * lane < kdim ? 4 * lane : 0;
 #pragma unroll
-        for (int a = 0; a < RW; ++a) wd[a] = ld_w4(wr[a] + e);
+        for (int a = 0; a < RW; ++a) wd[a] = ld_w4raw(wr[a] + e);
 #pragma unroll
         for (int b = 0; b < TW; ++b) xd[b] = *(const float4 *) (xr[b] + e);
     };
-    auto fma_step = [&](int i, const float4 (&wd)[RW], const float4 (&xd)[TW]) {
+    auto fma_step = [&](int i, const WR (&wd)[RW], const float4 (&xd)[TW]) {
         if (i >= niter || 256 * i + 4 * lane >= kdim) return;
 #pragma unroll
-        for (int a = 0; a < RW; ++a)
+        for (int a = 0; a < RW; ++a) {
+            const float4 wv = widen(wd[a]);
 #pragma unroll
             for (int b = 0; b < TW; ++b) {
                 float s = acc[a][b];
-                s = __builtin_fmaf(wd[a].x, xd[b].x, s);
-                s = __builtin_fmaf(wd[a].y, xd[b].y, s);
-                s = __builtin_fmaf(wd[a].z, xd[b].z, s);
-                s = __builtin_fmaf(wd[a].w, xd[b].w, s);
+                s = __builtin_fmaf(wv.x, xd[b].x, s);
+                s = __builtin_fmaf(wv.y, xd[b].y, s);
+                s = __builtin_fmaf(wv.z, xd[b].z, s);
+                s = __builtin_fmaf(wv.w, xd[b].w, s);
                 acc[a][b] = s;
             }
+        }
     };
     ld(0, wa, xa);
     for (int i = 0; i < niter; i += 2) {
@@ -160,28 +164,29 @@ __device__ __forceinline__ void gemv_block_lds(const WT *__restrict__ W, int row
         if (k < NW) { const int r = r0 + row; wsrc[k] = W + (size_t) (r < rows ? r : rows - 1) * kdim + 4 * lane; }
         else { const int t = t0 + row - GL_R; xsrc[k - NW] = x + (size_t) (t < nt ? t : nt - 1) * xs + 4 * lane; }
     }
-    auto ld = [&](int k, int e) -> f4v {
-        if (k < NW) { const float4 v = ld_w4(wsrc[k] + e); return f4v{v.x, v.y, v.z, v.w}; }
-        return *(const f4v *) (xsrc[k - NW] + e);
+    typename W4Raw<WT>::T prew[NW];   // the next step's loads (bf16 weights widened where they go to LDS)
+    f4v prex[NS - NW];
+    auto ld_all = [&](int e) {
+#pragma clang loop unroll(full)
+        for (int k = 0; k < NW; ++k) prew[k] = ld_w4raw(wsrc[k] + e);
+#pragma clang loop unroll(full)
+        for (int k = 0; k < NS - NW; ++k) prex[k] = *(const f4v *) (xsrc[k] + e);
     };
     float acc[RW][TW];
 #pragma unroll
     for (int a = 0; a < RW; ++a)
 #pragma unroll
         for (int b = 0; b < TW; ++b) acc[a][b] = 0.0f;
-    f4v pre[NS];
-#pragma clang loop unroll(full)
-    for (int k = 0; k < NS; ++k) pre[k] = ld(k, 0);
+    ld_all(0);
     const int niter = kdim / 256;
     for (int i = 0; i < niter; ++i) {
         __syncthreads();   // the previous step's reads of st are done
 #pragma clang loop unroll(full)
-        for (int k = 0; k < NS; ++k) st[tid + GL_THREADS * k] = pre[k];
-        __syncthreads();
-        if (i + 1 < niter) {
+        for (int k = 0; k < NW; ++k) { const float4 v = widen(prew[k]); st[tid + GL_THREADS * k] = f4v{v.x, v.y, v.z, v.w}; }
 #pragma clang loop unroll(full)
-            for (int k = 0; k < NS; ++k) pre[k] = ld(k, 256 * (i + 1));
-        }
+        for (int k = NW; k < NS; ++k) st[tid + GL_THREADS * k] = prex[k - NW];
+        __syncthreads();
+        if (i + 1 < niter) ld_all(256 * (i + 1));
         f4v xv[TW];
 #pragma unroll
         for (int b = 0; b < TW; ++b) xv[b] = st[(GL_R + TW * (wave >> 2) + b) * 64 + lane];
@@ -304,6 +309,7 @@ __global__ __launch_bounds__(RR_THREADS, 2) void k_router_rows(const WT *__restr
     dma_chunk(0, 0);
     // the weights in K order (the first half of every row, then the second): chunk 0's fmas over the first half run
     // while the second half is still on its way
+    typename W4Raw<WT>::T wl[RR_ROWS][NI];   // as loaded; widened (bf16) into w when the half has landed
     f4v w[RR_ROWS][NI];
     const WT *wr[RR_ROWS];
 #pragma unroll
@@ -311,7 +317,16 @@ __global__ __launch_bounds__(RR_THREADS, 2) void k_router_rows(const WT *__restr
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int a = 0; a < RR_ROWS; ++a) { const float4 v = ld_w4(wr[a] + 256 * i); w[a][i] = f4v{v.x, v.y, v.z, v.w}; }
+        for (int a = 0; a < RR_ROWS; ++a) wl[a][i] = ld_w4raw(wr[a] + 256 * i);
+    auto widen_half = [&](int h) {
+#pragma unroll
+        for (int ii = 0; ii < NI / 2; ++ii)
+#pragma unroll
+            for (int a = 0; a < RR_ROWS; ++a) {
+                const float4 v = widen(wl[a][h * (NI / 2) + ii]);
+                w[a][h * (NI / 2) + ii] = f4v{v.x, v.y, v.z, v.w};
+            }
+    };
     float acc[RR_ROWS][RR_TC];
     // the fmas of K half h (i in [h NI / 2, (h + 1) NI / 2)) of a chunk staged in buffer buf: each (row, token) chain
     // runs over i in order, so the halves in turn give the same bits as one pass
@@ -345,8 +360,10 @@ __global__ __launch_bounds__(RR_THREADS, 2) void k_router_rows(const WT *__restr
     for (int a = 0; a < RR_ROWS; ++a)
 #pragma unroll
         for (int u = 0; u < RR_TC; ++u) acc[a][u] = 0.0f;
+    widen_half(0);
     fma_half(0, 0);
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the second half
+    widen_half(1);
     if (nchunk > 1) dma_chunk(1, 1);
     constexpr int NOUT = RR_ROWS * RR_TC, P = 16, LPO = 64 / P, SUB = 64 / LPO;   // the tree of gemv_block_lds, 16 outputs a pass
     static_assert(NOUT % P == 0 && RR_WAVES * 64 * P <= RR_TC * ROWF4 * 4, "the passes fit a chunk buffer");
@@ -507,17 +524,18 @@ __global__ __launch_bounds__(64 * NW) void k_router_tile(const WT *__restrict__ 
     // the ring of four chunks on their way, in named slots of up to two float4 of A and of B (named variables: they
     // stay in registers)
     static_assert(NL == 1 || NL == 2, "one or two float4 of each operand a thread");
-    float4 sa0, sb0, ta0, tb0, sa1, sb1, ta1, tb1, sa2, sb2, ta2, tb2, sa3, sb3, ta3, tb3;
+    typename W4Raw<WT>::T sa0, ta0, sa1, ta1, sa2, ta2, sa3, ta3;   // weights as loaded (bf16 widened where they go to LDS)
+    float4 sb0, tb0, sb1, tb1, sb2, tb2, sb3, tb3;
 #define HY_RT_LOAD(c, SA, SB, TA, TB)                                                              \
     {                                                                                            \
-        SA = ld_w4(ga[0] + RT_KC * (c)); SB = *(const float4 *) (gb[0] + RT_KC * (c));           \
-        if constexpr (NL == 2) { TA = ld_w4(ga[NL - 1] + RT_KC * (c)); TB = *(const float4 *) (gb[NL - 1] + RT_KC * (c)); } \
+        SA = ld_w4raw(ga[0] + RT_KC * (c)); SB = *(const float4 *) (gb[0] + RT_KC * (c));           \
+        if constexpr (NL == 2) { TA = ld_w4raw(ga[NL - 1] + RT_KC * (c)); TB = *(const float4 *) (gb[NL - 1] + RT_KC * (c)); } \
     }
 #define HY_RT_STORE(buf, SA, SB, TA, TB)                                                           \
     {                                                                                            \
-        *(float4 *) &As[buf][lr * RT_LD + lc] = SA; *(float4 *) &Bs[buf][lr * RT_LD + lc] = SB;  \
+        *(float4 *) &As[buf][lr * RT_LD + lc] = widen(SA); *(float4 *) &Bs[buf][lr * RT_LD + lc] = SB;  \
         if constexpr (NL == 2) {                                                                 \
-            *(float4 *) &As[buf][(lr + RS) * RT_LD + lc] = TA; *(float4 *) &Bs[buf][(lr + RS) * RT_LD + lc] = TB; \
+            *(float4 *) &As[buf][(lr + RS) * RT_LD + lc] = widen(TA); *(float4 *) &Bs[buf][(lr + RS) * RT_LD + lc] = TB; \
         }                                                                                        \
     }
     f32x4 acc[2][TJ];
