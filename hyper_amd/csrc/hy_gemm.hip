@@ -1370,6 +1370,10 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     }
                 }
             }
+            // the next step's stage has landed (this wave's DMAs; the barrier at its top covers the others'): waited for
+            // here, ahead of the item's stores, so that no step waits for stores just issued (waited for at the next
+            // step's top: 131 MXFP4 tokens of 4096 x 2048, 8 experts, 116 us, here 113; 2048 Q5_K/Q6_K tokens 654, 645)
+            wait_vm<(D - 2) * C::L>();
             if (b != nsb - 1) return;
             // ---- the item's outputs, through this stage (every wave has finished reading it after a barrier), TOKP
             // tokens a pass: the waves' accumulators go there token-major -- rows padded by one float against bank
@@ -1419,8 +1423,8 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             if (nsteps > 1) { issue_raw(1); next_a(); }
             rl.load(raw_a(0), wave);
             rl.store(al_a(0), wave);
+            wait_vm<0>();
             for (int st = 0, it = 0, b = 0; st < nsteps; ++st) {
-                wait_vm<0>();
                 lds_barrier();   // weights st, raw rows st + 1 and aligned rows st are in place; step st - 1 is done with its own
                 const bool more = st + 1 < nsteps;
                 if (more) {
@@ -1450,8 +1454,8 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
         };
 #pragma unroll
         for (int s = 0; s < D - 1; ++s) issue();
+        wait_vm<(D - 2) * C::L>();
         for (int st = 0, it = 0, b = 0, stage = 0; st < nsteps; ++st) {
-            wait_vm<(D - 2) * C::L>();
             lds_barrier();
             issue();
             compute(it, b, stage, ntok);
