@@ -730,16 +730,19 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
 
 // IQ2_XS step on the 16x16x64 MFMA.  Lane quarter q's 16 values of MFMA j (64 j + 16 q ..) are scale group 4 j + q: the
 // two 8-groups of the 32-bit word qs[8 j + 2 q], qs[8 j + 2 q + 1] (9 bits of grid row, 7 of sign index each), scale
-// s = 2 nibble + 1 in 1 .. 31.  The codebook has three levels, 8 = 8 1 + 9 0, 25 = 8 2 + 9 1 and 43 = 8 2 + 9 3, so
-// B = sign s level splits into two int8 planes, B = 8 P + Q with P = sign s {1, 2, 2}, |P| <= 62, and Q = sign s {0, 1, 3},
-// |Q| <= 93: sum_g s_g dot_g = 8 X.P + 9 X.Q exactly.  A plane's byte is one of six per scale group (level, sign), held
-// in two registers, and v_perm picks four at a time: the LDS tables give each 8-group's levels and signs as nibbles
-// (iq2_sel_table: entry g the levels of row g, entry 512 + i the signs of sign index i in bit 2 of each nibble; value v
-// of the 8-group in byte v % 4, nibble v / 4), OR-ed into the selectors.  It replaced the generic step (two masked
-// 16x16x32 MFMAs a 32-value chunk, eight 24-bit multiply-adds an output column, 8-byte codebook and sign rows): the
-// 2048-token, 384-expert layer of d 7168, ff 2048, top-6: gate/up 3.95 -> 2.15 ms, down 2.05 -> 1.04 ms.  Bound by VALU
-// issue (75 % of the cycles at 16 waves, 290 instructions a wave and step; LDS 50 %, MFMA 20 %).
-constexpr int IQ2_SEL = 512 + 128;
+// s = 2 nibble + 1 in 1 .. 31.  The codebook has three levels, 8, 25 and 43, so a value of the group is one of the six v =
+// +-s level, |v| <= 1333, and B = v splits into two int8 planes, v = 16 P + Q with |P| <= 83 and -8 <= Q < 8: sum_g s_g
+// dot_g = 16 X.P + X.Q exactly.  A plane's six bytes per scale come from a 16-entry LDS table (one read without bank
+// conflicts; multiplied and negated in registers they cost seven more operations a group), and v_perm picks four at a
+// time: the selector table gives each 8-group's levels and signs as nibbles (iq2_sel_table: entry g the levels of row g,
+// entry 512 + i the signs of sign index i in bit 2 of each nibble; value v of the 8-group in byte v % 4, nibble v / 4),
+// OR-ed into the selectors.  Both tables lie in the first 64 KB of LDS, so that a lookup's base is the instruction's
+// offset and not an addition.  It replaced the generic step (two masked 16x16x32 MFMAs a 32-value chunk, eight 24-bit
+// multiply-adds an output column, 8-byte codebook and sign rows): the 2048-token, 384-expert layer call of d 7168, ff
+// 2048, top-6: 6.29 -> 3.51 ms, and 3473 -> 3294 us with the plane table, the 16 : 1 split and the offsets (55 of 290
+// operations a wave and step less).  VALU issue and the LDS pipe bound it about alike.
+constexpr int IQ2_SEL = 512 + 128, IQ2_TAB = 4 * IQ2_SEL + 16 * 16;   // selectors (dwords); bytes with the plane table
+static_assert(IQ2_TAB % 256 == 0, "the stages behind it stay at multiples of 256");
 __device__ __forceinline__ void iq2_sel_table(uint32_t *sel) {
     for (int i = threadIdx.x; i < IQ2_SEL; i += blockDim.x) {
         uint32_t v = 0, c = i < 512 ? c_iq2xs_code[i] : ksign((uint32_t) i - 512);
@@ -750,6 +753,16 @@ __device__ __forceinline__ void iq2_sel_table(uint32_t *sel) {
             v |= n << (8 * (j & 3) + 4 * (j >> 2));
         }
         sel[i] = v;
+    }
+    if (const int i = threadIdx.x; i < 16) {   // plane bytes of scale nibble i: P of the levels, of their negatives, Q likewise
+        uint32_t e[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+            const int l = n % 3, v = (n < 3 ? 1 : -1) * (2 * i + 1) * (l == 0 ? 8 : l == 1 ? 25 : 43), P = (v + 8) >> 4;
+            e[n / 3] |= (uint32_t) (P & 255) << (8 * l);
+            e[2 + n / 3] |= (uint32_t) ((v - 16 * P) & 255) << (8 * l);
+        }
+        ((uint4 *) (sel + IQ2_SEL))[i] = make_uint4(e[0], e[1], e[2], e[3]);
     }
 }
 // 4 bytes at p, which is 2-byte aligned (sb = p & 3 is 0 or 2): two aligned dwords from p - sb, joined.  (One unaligned
@@ -771,7 +784,7 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
     uint32_t w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) w[j] = ld4_u2(blk + 2 + 16 * j + 4 * q, al);
-    const uint32_t sc0 = ld4_u2(blk + 66, al) >> (4 * q), sc1 = ld4_u2(blk + 70, al) >> (4 * q);   // group 4 j + q: nibble 0 / 4
+    const uint32_t sc0 = ld4_u2(blk + 66, al), sc1 = ld4_u2(blk + 70, al);   // group 4 j + q: nibble 4 (j & 1) + q
     const float d = h2f(ld_u16(blk)) * 0.125f;
     const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * (q ^ rr);   // token row rr of tile 0, piece q
     const v4i z = {0, 0, 0, 0};
@@ -784,12 +797,13 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
         gb[j] = sel[__builtin_amdgcn_ubfe(w[j], 16, 9)];
         sb[j] = sel[512 + (w[j] >> 25)];
     }
+    auto planes = [&](int j) { return ((const uint4 *) (sel + IQ2_SEL))[__builtin_amdgcn_ubfe(j < 2 ? sc0 : sc1, 4 * q + 16 * (j & 1), 4)]; };
+    uint4 pl = planes(0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const uint32_t ca = ga[j] | sa[j], cb = gb[j] | sb[j];
-        const uint32_t s = 2 * (((j < 2 ? sc0 : sc1) >> (16 * (j & 1))) & 15) + 1, s2 = s | (s << 16);
-        const uint32_t Pp = (uint32_t) mul_bytes(0x00020201u, s2), Qp = (uint32_t) mul_bytes(0x00030100u, s2);
-        const uint32_t Pn = (Pp ^ 0x00FFFFFFu) + 0x00010101u, Qn = (Qp ^ 0x00FFFF00u) + 0x00010100u;   // the negated bytes
+        const uint32_t Pp = pl.x, Pn = pl.y, Qp = pl.z, Qn = pl.w;
+        if (j < 3) pl = planes(j + 1);
         const uint32_t i0 = ca & 0x07070707u, i1 = (ca >> 4) & 0x07070707u, i2 = cb & 0x07070707u, i3 = (cb >> 4) & 0x07070707u;
         const v4i BP = {(int) __builtin_amdgcn_perm(Pn, Pp, i0), (int) __builtin_amdgcn_perm(Pn, Pp, i1),
                         (int) __builtin_amdgcn_perm(Pn, Pp, i2), (int) __builtin_amdgcn_perm(Pn, Pp, i3)};
@@ -808,7 +822,7 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
     for (int t = 0; t < NT; ++t) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int si = ((dp[t][v] + dq[t][v]) << 3) + dq[t][v];
+            const int si = (dp[t][v] << 4) + dq[t][v];
             acc[T0 + t][v] = __builtin_fmaf(yd[(T0 + t) * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[T0 + t][v]);
         }
     }
@@ -1109,12 +1123,15 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     constexpr bool A0 = C::A0;
     constexpr int D = C::D, AQ = C::AROW;
     // stage s at s * SB: weights [wave][TB], activations [64][256], d [64]; A0: weights only, then the raw and aligned buffers
-    __shared__ __align__(256) uint8_t smem[C::SMEM];
+    // IQ2_XS: its tables first, where an LDS instruction's 16-bit offset reaches them (a lookup's address is then its index)
+    constexpr int TAB = T == IQ2_XS ? IQ2_TAB : 0;
+    __shared__ __align__(256) uint8_t smem0[TAB + C::SMEM];
+    uint8_t *const smem = smem0 + TAB;
     __shared__ uint64_t s_scan[1024 + C::WAVES];                // per expert group: exclusive prefix of its items per tile class
     __shared__ int s_item[C::ITEMS][3];                  // first pair in order, tokens, weight slot
     __shared__ int s_pair[C::ITEMS][GM_TOK];             // pair index of each token of the segment's items
     __shared__ float s_wt[GU ? 1 : C::ITEMS][GM_TOK];    // down: their route weights
-    __shared__ uint2 grid[T == IQ2_XS ? IQ2_SEL / 2 : iq2_lds(T)];   // the codebook (IQ2_XS: its selector table)
+    __shared__ uint2 grid[T == IQ2_XS ? 1 : iq2_lds(T)];   // the codebook
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, rr = lane & 15, q = lane >> 4;
     const int na = order_n[1];
     // ---- items.  Expert group g (cnt tokens) owns ceil(cnt / 64) items: full ones of 4 token tiles and a last one of
@@ -1145,7 +1162,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
         uint64_t ex = base + inc - loc;
 #pragma unroll
         for (int i = 0; i < C::PER; ++i) { s_scan[C::PER * tid + i] = ex; ex += c2[i]; }
-        if constexpr (T == IQ2_XS) iq2_sel_table((uint32_t *) grid);
+        if constexpr (T == IQ2_XS) iq2_sel_table((uint32_t *) smem0);
         else if constexpr (iq2_type(T)) expand_iq2_grid<T>(grid);
         __syncthreads();
     }
@@ -1335,7 +1352,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                 }
             } else if constexpr (T == IQ2_XS) {
                 const uint8_t *wt = stage_w(stage) + wave * C::TB;
-                const uint32_t *sel = (const uint32_t *) grid;
+                const uint32_t *sel = (const uint32_t *) smem0;
                 if (b == 0) {
                     switch (ntile) {
                     case 1: step_iq2xs<1, 0, true>(wt, as, yd, sel, acc); break;
