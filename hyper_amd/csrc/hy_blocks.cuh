@@ -138,7 +138,7 @@ template <> struct Item<Q2_K> {
             sb = sdot4((q[4 + i] >> sh) & 0x03030303u, ya[4 + i], sb);
         }
         const int16_t *bs = (const int16_t *) (y + 260);
-        si = (int) (scm & 15) * sa + (int) ((scm >> 8) & 15) * sb;
+        si = __mul24((int) (scm & 15), sa) + __mul24((int) ((scm >> 8) & 15), sb);   // exact: |sa| < 2^16
         sm = (int) ((scm >> 4) & 15) * bs[2 * L] + (int) (scm >> 12) * bs[2 * L + 1];
     }
     __device__ __forceinline__ float tval(int si, int sm) const {
@@ -170,7 +170,7 @@ template <> struct Item<IQ3_XXS> {
             s = sdot4(apply_mask(grid[(gw >> sh) & 255].x, m.x), ya[2 * l], s);
             s = sdot4(apply_mask(grid[(gw >> (sh + 8)) & 255].x, m.y), ya[2 * l + 1], s);
         }
-        si = (2 * (int) (a >> 28) + 1) * s;
+        si = __mul24(2 * (int) (a >> 28) + 1, s);   // exact: |s| <= 32 62 128
         sm = 0;
     }
     __device__ __forceinline__ float tval(int si, int) const { return (h2f(d) * 0.25f) * (float) si; }
@@ -199,7 +199,7 @@ template <> struct Item<IQ1_S> {
         }
         const int ls = 2 * (int) ((qh >> 12) & 7) + 1;
         const int16_t *bs = (const int16_t *) (y + 260);
-        si = ls * s;
+        si = __mul24(ls, s);   // exact: |s| <= 32 128
         sm = (qh & 0x8000 ? -ls : ls) * (bs[2 * L] + bs[2 * L + 1]);
     }
     __device__ __forceinline__ float tval(int si, int sm) const { return (h2f(d) * 0.125f) * (float) (8 * si + sm); }
@@ -226,7 +226,7 @@ template <> struct Item<IQ2_S> {
             const uint2 g = grid[((gq >> (8 * l)) & 255) | (((hs >> (2 * l)) & 3) << 8)], m = grid[1024 + ((sg >> (8 * l)) & 255)];
             s[l] = sdot4(apply_mask(g.y, m.y), ya[2 * l + 1], sdot4(apply_mask(g.x, m.x), ya[2 * l], 0));
         }
-        si = (2 * (int) ((hs >> 8) & 15) + 1) * (s[0] + s[1]) + (2 * (int) ((hs >> 12) & 15) + 1) * (s[2] + s[3]);
+        si = __mul24(2 * (int) ((hs >> 8) & 15) + 1, s[0] + s[1]) + __mul24(2 * (int) ((hs >> 12) & 15) + 1, s[2] + s[3]);   // exact: sums under 16 43 128
         sm = 0;
     }
     __device__ __forceinline__ float tval(int si, int) const { return (h2f(d) * 0.125f) * (float) si; }
@@ -259,7 +259,7 @@ template <> struct Item<IQ3_S> {
             s = sdot4(apply_mask(grid[i1].x, m.x), ya[2 * l], s);
             s = sdot4(apply_mask(grid[i2].x, m.y), ya[2 * l + 1], s);
         }
-        si = (2 * (int) (hs >> 8) + 1) * s;
+        si = __mul24(2 * (int) (hs >> 8) + 1, s);   // exact: |s| <= 32 15 128
         sm = 0;
     }
     __device__ __forceinline__ float tval(int si, int) const { return h2f(d) * (float) si; }
@@ -351,7 +351,7 @@ template <> struct Item<IQ4_XS> {
 #pragma unroll
         for (int i = 0; i < 4; ++i) { s = sdot4(kv4(q[i] & 0x0F0F0F0Fu), ya[i], s); s = sdot4(kv4((q[i] >> 4) & 0x0F0F0F0Fu), ya[4 + i], s); }
         const int ls = ((sl >> (4 * (L & 1))) & 0xF) | ((((dsh >> 16) >> (2 * L)) & 3) << 4);
-        si = (ls - 32) * s;
+        si = __mul24(ls - 32, s);   // exact: |s| <= 32 127 128
         sm = 0;
     }
     __device__ __forceinline__ float tval(int si, int) const { return h2f(dsh & 0xffff) * (float) si; }
@@ -378,7 +378,7 @@ template <> struct Item<IQ2_XS> {
             const uint2 g = grid[q[l] & 511], sm = grid[512 + (q[l] >> 9)];
             s[l] = sdot4(apply_mask(g.y, sm.y), ya[2 * l + 1], sdot4(apply_mask(g.x, sm.x), ya[2 * l], 0));
         }
-        si = (2 * (sc & 15) + 1) * (s[0] + s[1]) + (2 * (sc >> 4) + 1) * (s[2] + s[3]);
+        si = __mul24(2 * (sc & 15) + 1, s[0] + s[1]) + __mul24(2 * (sc >> 4) + 1, s[2] + s[3]);   // exact: sums under 2^17
         sm = 0;
     }
     __device__ __forceinline__ float tval(int si, int) const { return (h2f(d) * 0.125f) * (float) si; }
@@ -404,7 +404,7 @@ template <> struct Item<IQ2_XXS> {
             const uint2 g = grid[(a0 >> (8 * l)) & 255], m = grid[256 + ((a1 >> (7 * l)) & 127)];
             s = sdot4(apply_mask(g.y, m.y), ya[2 * l + 1], sdot4(apply_mask(g.x, m.x), ya[2 * l], s));
         }
-        si = (2 * (int) (a1 >> 28) + 1) * s;
+        si = __mul24(2 * (int) (a1 >> 28) + 1, s);   // exact: |s| <= 32 43 128
         sm = 0;
     }
     __device__ __forceinline__ float tval(int si, int) const { return (h2f(d) * 0.125f) * (float) si; }

@@ -137,9 +137,10 @@ constexpr int HY_TILE = 16;
 __host__ __device__ constexpr size_t tiled_off(int row, int span, int nspan, int sb) {
     return ((size_t) (row >> 4) * nspan + span) * (size_t) (HY_TILE * sb) + (size_t) (row & 15) * sb;
 }
-// the same within one expert matrix of under 4 GiB (the launchers check), as a 32-bit offset
+// the same within one expert matrix of under 4 GiB (the launchers check), as a 32-bit offset.  24-bit multiplies (a 32-bit
+// one issues at a quarter of their rate): the tile's number and its bytes are below 2^24 in such a matrix.
 __device__ __forceinline__ uint32_t tiled_off32(int row, int span, int nspan, int sb) {
-    return ((uint32_t) (row >> 4) * (uint32_t) nspan + (uint32_t) span) * (uint32_t) (HY_TILE * sb) + (uint32_t) (row & 15) * (uint32_t) sb;
+    return __umul24(__umul24(row >> 4, nspan) + (uint32_t) span, HY_TILE * sb) + __umul24(row & 15, sb);
 }
 __host__ __device__ constexpr int span_bytes(int t) { return block_bytes(t) * (256 / block_elems(t)); }
 // a slot-table entry as every kernel takes it: a local expert index below n_local, else -1 (absent)

@@ -150,7 +150,7 @@ __device__ __forceinline__ float item_t(const Item<T> &it, const uint8_t *y, int
         return 0.0f;
     } else {
         int si = 0, sm = 0;
-        if (valid) it.ints(y + (size_t) gi * Q8K_BYTES, L, si, sm);
+        if (valid) it.ints(y + __umul24(gi, Q8K_BYTES), L, si, sm);   // (24 bits: see tiled_off32)
         si = group8_isum(si);
         sm = group8_isum(sm);
         if (valid && L == 0) tv_out[tv_idx] = it.tval(si, sm);
@@ -171,7 +171,7 @@ __device__ __forceinline__ void item_t_all(const Item<T> &it, const uint8_t *y, 
         if (valid) tv_out[tv_idx + L] = v;
     } else {
         int si = 0, sm = 0;
-        it.ints(y + (size_t) gs * Q8K_BYTES, L, si, sm);
+        it.ints(y + __umul24(gs, Q8K_BYTES), L, si, sm);
         si = group8_isum(si);
         sm = group8_isum(sm);
         if (valid && L == 0) tv_out[tv_idx] = it.tval(si, sm);
@@ -241,8 +241,12 @@ constexpr int DEC_PIPE_NP = HY_DEC_PIPE_NP;        // passes per round when a wa
 // HQ: the block's 8 rw = 32 rows form one Q8_0 block of every pair's hidden row, and the fold also writes it to hq
 // (the down kernel then reads the hidden quantized instead of quantizing it in every block).  PIPE: for waves with
 // several rounds of items, each round's loads go out before the previous round's dots.
+// The one-round grid of DEC_GU_BLOCKS is three blocks a CU, six waves a SIMD, if the kernel takes at most 80 registers.
+// IQ4_XS comes to 82 by itself and fits 80 without spilling (except with the routing of 65-128 and of 513-1024 experts):
+// 184 against 155 us for one token through four layers (d 4096, 288 experts, ff 1536); the other types spill or fit.
+template <int T, int V> constexpr int dec_gu_waves() { return T == IQ4_XS && V != 2 && V != 16 ? 6 : 1; }
 template <int T, int V, int NP, bool HQ = false, bool PIPE = false>
-__global__ __launch_bounds__(64 * DEC_GU_WAVES) void k_route_gate_up(hy_moe_dev m, const float *__restrict__ logits, int ls, int ne, int k,
+__global__ __launch_bounds__(64 * DEC_GU_WAVES, (dec_gu_waves<T, V>())) void k_route_gate_up(hy_moe_dev m, const float *__restrict__ logits, int ls, int ne, int k,
                                                                    const uint8_t *__restrict__ xq, int *__restrict__ ids,
                                                                    float *__restrict__ wts, float *__restrict__ sg, float *__restrict__ h,
                                                                    int rw, int q8, int r8, uint8_t *__restrict__ hq) {
@@ -371,8 +375,8 @@ __global__ __launch_bounds__(64 * DEC_GU_WAVES) void k_route_gate_up(hy_moe_dev 
             const int r = cc.s, gi = cc.u, blk = block_elems(T) == 32 ? 8 * gi : gi;
             const bool valid = gi < ng && row0 + r < ff;
             if constexpr (iq2_type(T)) { bg[ps].grid = grid; bu[ps].grid = grid; }
-            item_t<T>(bg[ps], s_y, gi, L, valid, tw, r * rs + blk);
-            item_t<T>(bu[ps], s_y, gi, L, valid, tw, r * rs + nb + blk);
+            item_t<T>(bg[ps], s_y, gi, L, valid, tw, __mul24(r, rs) + blk);
+            item_t<T>(bu[ps], s_y, gi, L, valid, tw, __mul24(r, rs) + nb + blk);
             cc.next(rw, q8, r8);
         }
     };
@@ -529,7 +533,15 @@ __global__ __launch_bounds__(64 * DEC_DN_WAVES) void k_dec_down(hy_moe_dev m, co
     Cursor lc, cc;
     lc.start(g, ng);
     cc.start(g, ng);
+    // lane j: where pair j's matrix begins.  An item then costs two lane reads and a 24-bit multiply; from the slot it cost
+    // four 64-bit multiply-adds at a quarter of the rate.  With the 24-bit multiplies of the items: the 8-row IQ2_XS verify
+    // (d 7168, 384 experts, ff 2048, top-6) 265 -> 258 us, two rows of eight Q8_0 layers 279 -> 276.
+    const uint64_t my_base = (uint64_t) (my_slot >= 0 ? my_slot : 0) * m.down_bytes;
+    uint32_t okr = 0;   // bit ps: item ps of the round in `it` is there
     auto load_round = [&](int base) {
+        const uint64_t at = my_base + tiled_off(row, 0, ng, SPAN_W);   // (an offset: a pointer rebuilt from lane reads would load flat)
+        const uint32_t at_lo = (uint32_t) at, at_hi = my_slot >= 0 ? (uint32_t) (at >> 32) : ~0u;
+        okr = 0;
 #pragma unroll
         for (int ps = 0; ps < NP; ++ps) {
             const int i = base + g + 8 * ps;
@@ -538,8 +550,11 @@ __global__ __launch_bounds__(64 * DEC_DN_WAVES) void k_dec_down(hy_moe_dev m, co
                 if (i < items && row_ok && sl >= 0) it[ps].load(m.down + (size_t) sl * m.down_bytes + tiled_off(row, i, ng, SPAN_W), L);
             } else {
                 const int j = lc.u, gi = lc.s;
-                const int sl = __shfl(my_slot, j < 64 ? j : 0);
-                if (i < items && row_ok && sl >= 0) it[ps].load(m.down + (size_t) sl * m.down_bytes + tiled_off(row, gi, ng, SPAN_W), L);
+                const uint32_t lo = (uint32_t) __shfl((int) at_lo, j & 63), hi = (uint32_t) __shfl((int) at_hi, j & 63);
+                if (i < items && row_ok && (int) hi >= 0) {
+                    it[ps].load(m.down + (((uint64_t) hi << 32) | lo) + __umul24(gi, HY_TILE * SPAN_W), L);
+                    okr |= 1u << ps;
+                }
                 lc.next(ng, q8, r8);
             }
         }
@@ -597,8 +612,8 @@ __global__ __launch_bounds__(64 * DEC_DN_WAVES) void k_dec_down(hy_moe_dev m, co
                         item_t_all<T>(it[ps], hq + (size_t) j * ng * SPAN_L, i, L, i < items && pair_ok(j), tw, j * (nb | 1) + blk);
                 } else {
                     const int j = cc.u, gi = cc.s;
-                    const bool valid = i < items && pair_ok(j);
-                    item_t<T>(it[ps], hq + (size_t) j * ng * SPAN_L, gi, L, valid, tw, j * (nb | 1) + (block_elems(T) == 32 ? 8 * gi : gi));
+                    const bool valid = (okr >> ps) & 1;
+                    item_t<T>(it[ps], hq + __umul24(j, ng * SPAN_L), gi, L, valid, tw, __mul24(j, nb | 1) + (block_elems(T) == 32 ? 8 * gi : gi));
                     cc.next(ng, q8, r8);
                 }
             }
@@ -745,8 +760,8 @@ __global__ __launch_bounds__(64 * DEC_GU_WAVES) void k_shared_gate_up(hy_moe_dev
             for (int t = 0; t < SH_NT; ++t) {
                 if (t >= ntb) break;   // uniform (token 0 always runs: its weight-side work serves the others)
                 const uint8_t *yt = s_y + (size_t) t * ybytes;
-                item_t_all<T>(ig[ps], yt, gi, L, valid, tv, (t * RB + rr) * rs + blk);
-                item_t_all<T>(iu[ps], yt, gi, L, valid, tv, (t * RB + rr) * rs + nb + blk);
+                item_t_all<T>(ig[ps], yt, gi, L, valid, tv, __mul24(t * RB + rr, rs) + blk);
+                item_t_all<T>(iu[ps], yt, gi, L, valid, tv, __mul24(t * RB + rr, rs) + nb + blk);
             }
             cc.next(rw, q8, r8);
         }
