@@ -22,9 +22,31 @@ __global__ __launch_bounds__(256) void k_q8_0(const float *__restrict__ x, int x
     if (b >= nb) return;
     q8_0_pair_wave(x + (size_t) t * xs + 32 * b, q + ((size_t) t * nb + b) * Q8_0_BYTES, b + 1 < nb, Q8_0_BYTES, 2);
 }
+// The same blocks from 16-byte loads, eight lanes a block of 32 values (x 16-byte aligned, xs a multiple of 4): the scale's
+// two divisions are taken once for four values and a lane stores four bytes; a value a lane is bound by those operations
+// (18 us for 4072 rows of 1536; the 509-token IQ4_NL layer call with 288 experts 1077 -> 1066 us).
+__global__ __launch_bounds__(256) void k_q8_0v(const float *__restrict__ x, int xs, int nb, int nblk, uint8_t *__restrict__ q) {
+    const int u = blockIdx.x * 32 + (threadIdx.x >> 3), L = threadIdx.x & 7;
+    if (u >= nblk) return;   // uniform over the block's eight lanes
+    const int t = u / nb, b = u - t * nb;
+    const float4 v = *(const float4 *) (x + (size_t) t * xs + 32 * b + 4 * L);
+    float am = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    am = fmaxf(am, dpp_f<DPP_XOR1>(am));
+    am = fmaxf(am, dpp_f<DPP_XOR2>(am));
+    am = fmaxf(am, dpp_f<DPP_HALF_MIRROR>(am));
+    const float d = am / 127.f, id = am != 0.0f ? 127.f / am : 0.0f;
+    const uint32_t q0 = (uint8_t) (int8_t) (int) __builtin_rintf(v.x * id), q1 = (uint8_t) (int8_t) (int) __builtin_rintf(v.y * id);
+    const uint32_t q2 = (uint8_t) (int8_t) (int) __builtin_rintf(v.z * id), q3 = (uint8_t) (int8_t) (int) __builtin_rintf(v.w * id);
+    uint16_t *o = (uint16_t *) (q + (size_t) u * Q8_0_BYTES);
+    o[1 + 2 * L] = (uint16_t) (q0 | (q1 << 8));
+    o[2 + 2 * L] = (uint16_t) (q2 | (q3 << 8));
+    if (L == 0) o[0] = f2h(d);
+}
 int launch_q8(int vtype, const float *x, int xs, int n, int nt, void *q, hipStream_t s) {
     if (nt == 0) return HY_OK;
     if (vtype == Q8_K) hipLaunchKernelGGL(k_q8k, dim3((nt * (n / 256) + 15) / 16), dim3(256), 0, s, x, xs, n, nt, (uint8_t *) q);
+    else if (((uintptr_t) x & 15) == 0 && (xs & 3) == 0 && (size_t) nt * (n / 32) < (1u << 30))
+        hipLaunchKernelGGL(k_q8_0v, dim3((nt * (n / 32) + 31) / 32), dim3(256), 0, s, x, xs, n / 32, nt * (n / 32), (uint8_t *) q);
     else hipLaunchKernelGGL(k_q8_0, dim3((n / 32 + 7) / 8, nt), dim3(256), 0, s, x, xs, n, (uint8_t *) q);
     return check_launch("hy_q8_quantize");
 }
