@@ -1125,8 +1125,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     // stage s at s * SB: weights [wave][TB], activations [64][256], d [64]; A0: weights only, then the raw and aligned buffers
     // IQ2_XS: its tables first, where an LDS instruction's 16-bit offset reaches them (a lookup's address is then its index)
     constexpr int TAB = T == IQ2_XS ? IQ2_TAB : 0;
-    __shared__ __align__(256) uint8_t smem0[TAB + C::SMEM];
-    uint8_t *const smem = smem0 + TAB;
+    __shared__ __align__(256) uint8_t smem[TAB + C::SMEM];
     __shared__ uint64_t s_scan[1024 + C::WAVES];                // per expert group: exclusive prefix of its items per tile class
     __shared__ int s_item[C::ITEMS][3];                  // first pair in order, tokens, weight slot
     __shared__ int s_pair[C::ITEMS][GM_TOK];             // pair index of each token of the segment's items
@@ -1162,7 +1161,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
         uint64_t ex = base + inc - loc;
 #pragma unroll
         for (int i = 0; i < C::PER; ++i) { s_scan[C::PER * tid + i] = ex; ex += c2[i]; }
-        if constexpr (T == IQ2_XS) iq2_sel_table((uint32_t *) smem0);
+        if constexpr (T == IQ2_XS) iq2_sel_table((uint32_t *) smem);
         else if constexpr (iq2_type(T)) expand_iq2_grid<T>(grid);
         __syncthreads();
     }
@@ -1200,16 +1199,23 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     const int row = 16 * tile_row + rr;
     const uint8_t *Wmat = (GU ? (wave < C::HALF ? m.gate : m.up) : m.down) + (size_t) tile_row * nsb * C::TB;
     const size_t arow = (size_t) nsb * AQ;
-    auto stage_w = [&](int s) { return smem + s * C::SB; };
-    auto stage_a = [&](int s) { return (int8_t *) (smem + s * C::SB + C::WB); };
-    auto stage_d = [&](int s) { return (const float *) (smem + s * C::SB + C::WB + C::AB); };
-    auto raw_a = [&](int s) { return smem + D * C::SB + (s & 1) * C::RAW; };
-    auto al_a = [&](int s) { return smem + D * C::SB + 2 * C::RAW + (s & 1) * C::AL; };
+    // (offsets from the array itself: through a pointer variable behind the tables the types without tables were scheduled
+    // anew as well, and the 509-token IQ4_NL layer call took 1064 us instead of 1004)
+    auto stage_w = [&](int s) { return smem + TAB + s * C::SB; };
+    auto stage_a = [&](int s) { return (int8_t *) (smem + TAB + s * C::SB + C::WB); };
+    auto stage_d = [&](int s) { return (const float *) (smem + TAB + s * C::SB + C::WB + C::AB); };
+    auto raw_a = [&](int s) { return smem + TAB + D * C::SB + (s & 1) * C::RAW; };
+    auto al_a = [&](int s) { return smem + TAB + D * C::SB + 2 * C::RAW + (s & 1) * C::AL; };
 
     for (int seg = 0; seg < my_items; seg += C::ITEMS) {
         const int nit = min(C::ITEMS, my_items - seg);
         __syncthreads();   // readers of the previous segment's tables are done
-        for (int i = tid; i < nit; i += C::THREADS) {
+        // a thread id that the compiler cannot hoist out of the segment loop: kept live across the stream, the table
+        // addresses made from it went to scratch in the kernels near 128 registers (IQ4_NL, Q4_K gate/up), and a scratch
+        // reload is a vector memory operation that the compiler waits for by draining the stream
+        int ts = tid;
+        asm volatile("" : "+v"(ts));
+        for (int i = ts; i < nit; i += C::THREADS) {
             const int k = seg + i;
             int pos = k * ys + ((k & 1) ? ys - 1 - y0 : y0);   // position in the class order
             int cls = 0;                                        // field of s_scan: 0 = 4 tiles, 1 = 3, 2 = 2, 3 = 1
@@ -1227,7 +1233,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             s_item[i][2] = m.slot[egrp[3 * lo]];
         }
         __syncthreads();
-        for (int i = tid; i < nit * GM_TOK; i += C::THREADS) {
+        for (int i = ts; i < nit * GM_TOK; i += C::THREADS) {
             const int it = i / GM_TOK, tk = i - it * GM_TOK;
             const int pr = tk < s_item[it][1] ? order[s_item[it][0] + tk] : -1;
             s_pair[it][tk] = pr;
@@ -1352,7 +1358,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                 }
             } else if constexpr (T == IQ2_XS) {
                 const uint8_t *wt = stage_w(stage) + wave * C::TB;
-                const uint32_t *sel = (const uint32_t *) smem0;
+                const uint32_t *sel = (const uint32_t *) smem;
                 if (b == 0) {
                     switch (ntile) {
                     case 1: step_iq2xs<1, 0, true>(wt, as, yd, sel, acc); break;
@@ -1404,17 +1410,20 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             float *s_o = (float *) stage_w(stage);             // gate (or down) values
             float *s_u = s_o + TOKP * LD;                      // up values
             const int row0 = bx * OR;
+            // IQ4_NL is at its 128 registers: its epilogue makes its lane constants here instead of keeping them live across
+            // the stream (the other kernels have the registers, and are 1-3 % slower this way)
+            const int el = T == IQ4_NL ? lane_id_here() : lane, er = el & 15, eq = el >> 4;
             for (int p0 = 0; p0 < ntok; p0 += TOKP) {
                 lds_barrier();   // the stage (or the previous pass) is no longer read
                 {
                     float *dst = GU && wave >= C::HALF ? s_u : s_o;
-                    const int orow = (GU ? wave % C::HALF : wave) * 16 + rr;
+                    const int orow = (GU ? wave % C::HALF : wave) * 16 + er;
 #pragma unroll
                     for (int tile = 0; tile < GM_TILES; ++tile) {
                         if (tile >= ntile) break;
                         if (tile * 16 < p0 || tile * 16 >= p0 + TOKP) continue;
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) dst[(tile * 16 - p0 + 4 * q + v) * LD + orow] = acc[tile][v];
+                        for (int v = 0; v < 4; ++v) dst[(tile * 16 - p0 + 4 * eq + v) * LD + orow] = acc[tile][v];
                     }
                 }
                 lds_barrier();
@@ -1423,7 +1432,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                     const float wt = GU ? 0.0f : s_wt[GU ? 0 : it][tok];
                     const float *so = s_o + (tok - p0) * LD, *su = s_u + (tok - p0) * LD;
 #pragma unroll
-                    for (int r = lane; r < OR; r += 64) store_f32(o + r, GU ? hy_swiglu(so[r], su[r], m.clamp) : wt * so[r]);
+                    for (int r = el; r < OR; r += 64) store_f32(o + r, GU ? hy_swiglu(so[r], su[r], m.clamp) : wt * so[r]);
                 }
             }
         };
