@@ -835,27 +835,40 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
 // run-time tile loop took its branches at every chunk; without the empty asm on each sum the compiler regrouped the
 // chunks' sums and spilled.)  IQ4_XS, 1000 tokens, 288 experts, d 4096, ff 1536, top-8: the layer call 1252 -> 1125 us,
 // with the lds_at addresses and the geometry of g5_waves; bound by VALU issue (82 % of the cycles in gate/up).
+// One tile of a type with 16-value groups (G1) leaves most of the 256 registers free and is bound by latency: its operand
+// reads go out together and its chunks are scheduled as one piece; with one chunk in flight at a time a layer call of 37
+// tokens (d 2048, 64 experts, ff 768, top-8) took 130.5 us in Q2_K, 133 in Q3_K and 141 in IQ2_S, here 124, 123 and 131
+// (the run-time tile loop: 120, 127 and 136).
 template <int T, int NT, bool FIRST>
 __device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, const int8_t *as, const float *yd, float (&acc)[GM_TILES][4]) {
 #pragma unroll
     for (int t = NT; t < GM_TILES; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
-    constexpr bool G = Raw<T>::g16, MN = Raw<T>::mins;
-    const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
+    constexpr bool G = Raw<T>::g16, MN = Raw<T>::mins, G1 = G && NT == 1;
+    const int lid = G ? (int) (threadIdx.x & 63) : lane_id_here(), q = lid >> 4, rr = lid & 15;
     Raw<T> w;
     w.load(wt + rr * span_bytes(T), q);
     const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * ((q >> 1) ^ rr) + 8 * (q & 1);   // row rr of tile 0, chunk 0
     const v4i z = {0, 0, 0, 0};
-    constexpr int AHEAD = NT <= 2 ? 1 : 0;
+    // (two tiles of 16-value groups, and one whose values come from a table: 141 instead of 131 us for IQ2_S as above)
+    constexpr int AHEAD = G ? G1 && !iq2_type(T) : NT <= 2;
     v4i D[1 + AHEAD][NT], E[1 + AHEAD][NT], sm[NT];
     int s0[1 + AHEAD], s1[1 + AHEAD], si[NT][4];
+    constexpr int UP = G1 ? 8 : 1;   // chunks whose operands are read together
+    long Ac[UP][NT];
+    auto read = [&](int c) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) Ac[c % UP][t] = lds_at<long>((a0 ^ (32 * c)) + t * 16 * 256);
+    };
+    if constexpr (G1) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) read(c);
+    }
     auto mul = [&](int c) {
         const int s = AHEAD ? c & 1 : 0;
-        const uint32_t ac = a0 ^ (32 * c);
-        long A[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) A[t] = lds_at<long>(ac + t * 16 * 256);
+        if constexpr (!G1) read(c);
+        const long (&A)[NT] = Ac[c % UP];
         uint32_t b0, b1;
         int mn;
         w.chunk(c, q, grid, b0, b1, s0[s], s1[s], mn);
@@ -881,7 +894,7 @@ __device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, c
                 int x = c ? si[t][v] : 0;
                 x += __mul24(s0[s], D[s][t][v]);
                 if constexpr (G) x += __mul24(s1[s], E[s][t][v]);
-                asm volatile("" : "+v"(x));   // the chain of chunks is not regrouped (which kept every chunk's D live)
+                if constexpr (!G1) asm volatile("" : "+v"(x));   // the chain of chunks is not regrouped (which kept every chunk's D live)
                 si[t][v] = x;
             }
     };
@@ -890,7 +903,7 @@ __device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, c
     for (int c = 0; c < 8; ++c) {
         if constexpr (AHEAD) { if (c < 7) mul(c + 1); } else mul(c);
         scale(c);
-        asm volatile("");   // a scheduling-region boundary per chunk (register pressure)
+        if constexpr (!G1) asm volatile("");   // a scheduling-region boundary per chunk (register pressure)
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t)
