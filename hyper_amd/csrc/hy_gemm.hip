@@ -1743,18 +1743,37 @@ static bool a0_fits(int n_pairs, int k, int in_dim, int max_active) {
            max_items(n_pairs, max_active) < GM_MAX_ITEMS;
 }
 
+// One k_gemm launch: W waves a block, B blocks a CU (8 W output rows a block for gate/up, 16 W for down; ff and n are
+// multiples of 256, so 8 and 16 waves both tile them).
+template <int T, bool GU, int W, int B>
+static int launch_k_gemm(const hy_moe_dev &m, const void *a, int k, int n_pairs, const int *order, const int *order_n, const int *egrp,
+                         int max_active, const float *wts, float *out, hipStream_t s) {
+    const int rb = GU ? m.ff / (8 * W) : m.n / (16 * W);
+    dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, B == 1));   // two blocks a CU: every slot counts
+    hipLaunchKernelGGL((k_gemm<T, GU, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) a, div_mul_of(k), order, order_n, egrp, wts, out);
+    return check_launch(GU ? "hy_moe_gemm_gate_up" : "hy_moe_gemm_down");
+}
+// The same, in 8-wave blocks where blocks of 16 waves would take at most half of the CUs: twice the blocks then still run
+// at once, each with half of the weight rows to stream and decode.  d 2048, ff 1024, one expert and 64 tokens: IQ4_NL 97
+// -> 76 us, MXFP4 100 -> 79, IQ2_XS 81 -> 69, IQ4_XS 72 -> 68; 8 experts, top-2, 64 tokens: 81 -> 65, 80 -> 67, 72 -> 61
+// and 64 -> 61, Q4_K/Q6_K 68 -> 63.  Past the half the 16-wave blocks win: 512 of those tokens (192 blocks of 16 waves)
+// in IQ2_XS 91 us, in 8-wave blocks 96.
+template <int T, bool GU, int W, int B>
+static int launch_k_gemm_fit(const hy_moe_dev &m, const void *a, int k, int n_pairs, const int *order, const int *order_n, const int *egrp,
+                             int max_active, const float *wts, float *out, hipStream_t s) {
+    if constexpr (W == 16) {
+        if (2 * max_items(n_pairs, max_active) * (GU ? m.ff / 128 : m.n / 256) <= cu_count())
+            return launch_k_gemm<T, GU, 8, B>(m, a, k, n_pairs, order, order_n, egrp, max_active, wts, out, s);
+    }
+    return launch_k_gemm<T, GU, W, B>(m, a, k, n_pairs, order, order_n, egrp, max_active, wts, out, s);
+}
+
 int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs, const int *order, const int *order_n, const int *egrp,
                         int max_active, float *h, hipStream_t s) {
     if (max_active <= 0 || n_pairs <= 0) return HY_OK;
     if (vec_dot_type(m.tg) == Q8_0) {
         if (a0_fits(n_pairs, k, m.n, max_active)) {
-            HY_A0_SWITCH(m.tg, {
-                constexpr int W = a0_waves(TT);
-                const int rb = m.ff / (8 * W);
-                dim3 grid(rb, item_slots(rb, n_pairs, max_active, 1, true));
-                hipLaunchKernelGGL((k_gemm<TT, true, W, 1>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
-                return check_launch("hy_moe_gemm_gate_up");
-            });
+            HY_A0_SWITCH(m.tg, return (launch_k_gemm_fit<TT, true, a0_waves(TT), 1>(m, xq, k, n_pairs, order, order_n, egrp, max_active, nullptr, h, s)));
         }
         const int rt = (m.ff + 31) / 32;
         dim3 grid(rt, item_slots(rt, n_pairs, max_active, 3));
@@ -1772,31 +1791,16 @@ int launch_gemm_gate_up(const hy_moe_dev &m, const void *xq, int k, int n_pairs,
     // the rest to them (the 2048-token Q5_K/Q6_K chunk 690 -> 683 us; alone it takes 46 us against 32 at 8 waves and
     // twice the blocks).  Other small grids keep 8 waves.  ff is a multiple of 256, so either size tiles it.
     if (m.tg == Q5_K && (max_items(n_pairs, max_active) * (m.ff / 128) >= cu_count() || max_active == 1)) {
-        const int rb = m.ff / 128;
-        dim3 grid(rb, item_slots(rb, n_pairs, max_active, 1, true));
-        hipLaunchKernelGGL((k_gemm<Q5_K, true, 16, 1>), grid, dim3(1024), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
-        return check_launch("hy_moe_gemm_gate_up");
+        return launch_k_gemm<Q5_K, true, 16, 1>(m, xq, k, n_pairs, order, order_n, egrp, max_active, nullptr, h, s);
     }
-    HY_GEMM_SWITCH(m.tg, {
-        constexpr int W = g5_waves<TT, true>(), B = g5_blocks<TT, true>();
-        const int rb = m.ff / (8 * W);   // 8 W output rows a block
-        dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, B == 1));   // two blocks a CU: every slot counts
-        hipLaunchKernelGGL((k_gemm<TT, true, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) xq, div_mul_of(k), order, order_n, egrp, nullptr, h);
-        return check_launch("hy_moe_gemm_gate_up");
-    });
+    HY_GEMM_SWITCH(m.tg, return (launch_k_gemm_fit<TT, true, g5_waves<TT, true>(), g5_blocks<TT, true>()>(m, xq, k, n_pairs, order, order_n, egrp, max_active, nullptr, h, s)));
 }
 int launch_gemm_down(const hy_moe_dev &m, const void *hq, int n_pairs, const int *order, const int *order_n, const int *egrp, int max_active,
                      const float *wts, float *y, hipStream_t s) {
     if (max_active <= 0 || n_pairs <= 0) return HY_OK;
     if (vec_dot_type(m.td) == Q8_0) {
         if (a0_fits(n_pairs, 1, m.ff, max_active)) {
-            HY_A0_SWITCH(m.td, {
-                constexpr int W = a0_waves(TT);
-                const int rb = m.n / (16 * W);
-                dim3 grid(rb, item_slots(rb, n_pairs, max_active, 1, true));
-                hipLaunchKernelGGL((k_gemm<TT, false, W, 1>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) hq, div_mul_of(1), order, order_n, egrp, wts, y);
-                return check_launch("hy_moe_gemm_down");
-            });
+            HY_A0_SWITCH(m.td, return (launch_k_gemm_fit<TT, false, a0_waves(TT), 1>(m, hq, 1, n_pairs, order, order_n, egrp, max_active, wts, y, s)));
         }
         const int rt = (m.n + GM_ROWS - 1) / GM_ROWS;
         dim3 grid(rt, item_slots(rt, n_pairs, max_active, 3));
@@ -1807,13 +1811,7 @@ int launch_gemm_down(const hy_moe_dev &m, const void *hq, int n_pairs, const int
     }
     if ((size_t) n_pairs * (m.ff / 256) * Q8K_BYTES >= (1ull << 32)) { set_error("hy_moe_gemm_down: activations of 4 GB or more"); return HY_EBAD_SHAPE; }
     if (max_items(n_pairs, max_active) >= GM_MAX_ITEMS) { set_error("hy_moe_gemm_down: %d pairs make more than %d work items", n_pairs, GM_MAX_ITEMS - 1); return HY_EBAD_SHAPE; }
-    HY_GEMM_SWITCH(m.td, {
-        constexpr int W = g5_waves<TT, false>(), B = g5_blocks<TT, false>();
-        const int rb = m.n / (16 * W);   // 16 W output rows a block
-        dim3 grid(rb, item_slots(rb, n_pairs, max_active, B, true));
-        hipLaunchKernelGGL((k_gemm<TT, false, W, B>), grid, dim3(64 * W), 0, s, m, (const uint8_t *) hq, div_mul_of(1), order, order_n, egrp, wts, y);
-        return check_launch("hy_moe_gemm_down");
-    });
+    HY_GEMM_SWITCH(m.td, return (launch_k_gemm_fit<TT, false, g5_waves<TT, false>(), g5_blocks<TT, false>()>(m, hq, 1, n_pairs, order, order_n, egrp, max_active, wts, y, s)));
 }
 
 } // namespace hy
