@@ -25,11 +25,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ v4i mfma16(long a, long b, v4i c) { return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ long mk_long(uint32_t lo, uint32_t hi) { return (long) (((unsigned long long) hi << 32) | lo); }
-__device__ __forceinline__ uint2 load8_a2(const uint8_t *p) {   // 8 bytes from a 2-byte aligned address, no overread
-    if (((uintptr_t) p & 3) == 0) { const uint32_t *w = (const uint32_t *) p; return make_uint2(w[0], w[1]); }
-    const uint32_t h0 = *(const uint16_t *) p, d1 = *(const uint32_t *) (p + 2), h2 = *(const uint16_t *) (p + 6);
-    return make_uint2(h0 | (d1 << 16), (d1 >> 16) | (h2 << 16));
-}
 
 // Branch-free loads from 2-byte aligned addresses (a fixed instruction count per step lets the compiler count
 // the loads in flight): whole dwords from the aligned-down address, joined with v_alignbyte.
@@ -42,39 +37,13 @@ __device__ __forceinline__ uint2 ld8_2a(const uint8_t *p) {
     const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
     return make_uint2(join_b(d1, d0, sb), join_b(d2, d1, sb));
 }
-// 16 bytes at p (2-byte aligned), with p + 18 the end of the block: the fifth dword is read only when p is
-// misaligned (else the fourth is read again), so nothing past p + 18 is touched
-__device__ __forceinline__ uint4 ld16_2a_tail(const uint8_t *p) {
-    const uint32_t *w = (const uint32_t *) (p - ((uintptr_t) p & 3));
-    const uint32_t sb = (uint32_t) ((uintptr_t) p & 3);
-    const uint32_t d0 = w[0], d1 = w[1], d2 = w[2], d3 = w[3], d4 = w[sb ? 4 : 3];
-    return make_uint4(join_b(d1, d0, sb), join_b(d2, d1, sb), join_b(d3, d2, sb), join_b(d4, d3, sb));
-}
 
 // The raw bytes of one weight row's 256-value block that lane quarter q needs, and their decoding per 32-value
 // chunk c: B operand words b0/b1 (8 int8 values), scale(s), min.
 template <int T> struct Raw;
 
-template <> struct Raw<Q4_K> {   // 144 B: d, dmin, scales[12], qs[128]; chunk c: nibbles (c & 1) of qs[32 (c / 2) + 8 q ..]
-    static constexpr bool mins = true, g16 = false, per_chunk = false;
-    uint4 hd; uint2 qv[4];
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-        hd = load16_a4(blk);
-#pragma unroll
-        for (int jp = 0; jp < 4; ++jp) qv[jp] = *(const uint2 *) (blk + 16 + 32 * jp + 8 * q);
-    }
-    __device__ __forceinline__ void chunk(int c, int, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int sh = 4 * (c & 1);
-        b0 = (qv[c >> 1].x >> sh) & 0x0F0F0F0Fu; b1 = (qv[c >> 1].y >> sh) & 0x0F0F0F0Fu;
-        scale_min_k4(hd.y, hd.z, hd.w, c, s0, mn);
-        s1 = 0;
-    }
-    __device__ __forceinline__ float fold(int si, int sm) const {
-        return __builtin_fmaf(h2f(hd.x & 0xffff), (float) si, -(h2f(hd.x >> 16) * (float) sm));
-    }
-};
 template <> struct Raw<Q5_K> {   // 176 B: + qh[32] @16 (bit c of qh[l] is bit 4 of chunk c's value l), qs @48
-    static constexpr bool mins = true, g16 = false, per_chunk = false;
+    static constexpr bool mins = true, g16 = false;
     uint2 qv[4], qh; uint32_t dm, sl, sh, ml, mh;   // scales and mins of chunks 0..3 and 4..7, a byte each
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         const uint4 hd = load16_a4(blk);
@@ -104,7 +73,7 @@ template <> struct Raw<Q5_K> {   // 176 B: + qh[32] @16 (bit c of qh[l] is bit 4
 // 32 (c >> 2) + 8 q ..; the chunk's 16-groups 2 c (lanes q < 2) and 2 c + 1 (q >= 2): scales s0 / s1, and the lane's
 // own group's min (the mins MFMA takes each lane quarter's bytes, so each 8-value piece carries its group's min).
 template <> struct Raw<Q2_K> {
-    static constexpr bool mins = true, g16 = true, per_chunk = false;
+    static constexpr bool mins = true, g16 = true;
     uint4 scv; uint2 qv[2]; uint32_t dm;
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         scv = load16_a4(blk);
@@ -129,7 +98,7 @@ template <> struct Raw<Q2_K> {
 // halfword at 2 + 8 c + 2 q), sign index bits 7 q .. of the word at 66 + 4 c, the chunk's scale 2 sc + 1 (bits 28 ..)
 // (src/kernels4.cu:613-627; ggml's vec_dot_iq3_xxs_q8_K integers).
 template <> struct Raw<IQ3_XXS> {
-    static constexpr bool mins = false, g16 = false, per_chunk = false;
+    static constexpr bool mins = false, g16 = false;
     uint32_t gi[4], a[8], d;   // gi: the lane's index pair of chunk c in halfword c % 2 of gi[c / 2]
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -153,7 +122,7 @@ template <> struct Raw<IQ3_XXS> {
 // -1 / 0 / 1), the chunk's scale ls; the delta term rides on the mins MFMA with the chunk's ls * (+-1) as its "min", so
 // sm = sum_ib ls sign sum_32 y and the fold is (d / 8) (8 si + sm) (src/kernels4.cu:650-659; src/iq1s_dot.h:26-64).
 template <> struct Raw<IQ1_S> {
-    static constexpr bool mins = true, g16 = false, per_chunk = false;
+    static constexpr bool mins = true, g16 = false;
     uint32_t gq[2], qh[4], d;   // gq: the lane's index byte of chunk c in byte c % 4 of gq[c / 4]; qh[c] in halfwords
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         gq[0] = gq[1] = 0;
@@ -177,7 +146,7 @@ template <> struct Raw<IQ1_S> {
 // sign byte signs[4 c + q], the chunk's 16-group scales 2 sc + 1 from the nibbles of scales[c] (s0 for lanes q < 2)
 // (src/kernels4.cu:602-613; ggml's vec_dot_iq2_s_q8_K integers).
 template <> struct Raw<IQ2_S> {
-    static constexpr bool mins = false, g16 = true, per_chunk = false;
+    static constexpr bool mins = false, g16 = true;
     uint32_t gq[2], sg[2], qh[2], sc[2], d;   // byte c % 4 of [c / 4]: the lane's index byte, its sign byte, qh[c], scales[c]
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         gq[0] = gq[1] = sg[0] = sg[1] = 0;
@@ -210,7 +179,7 @@ template <> struct Raw<IQ2_S> {
 // 2 q, 2 q + 1 of qh[c] as their 9th bits, sign byte signs[4 c + q], the chunk's scale 2 sc + 1 (nibble c & 1 of
 // scales[c / 2]) (src/kernels4.cu:682-695; src/iq3s_dot.h:48-76 integers).
 template <> struct Raw<IQ3_S> {
-    static constexpr bool mins = false, g16 = false, per_chunk = false;
+    static constexpr bool mins = false, g16 = false;
     uint32_t gi[4], qh[2], sg[2], sc, d;   // gi: index pairs (halfword c % 2 of gi[c / 2]); qh, sg: byte c % 4 of [c / 4]
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -244,7 +213,7 @@ __device__ __forceinline__ int q3k_scale(const uint32_t (&s)[3], int is) {
     return (((byte(is & 7) >> (4 * (is >> 3))) & 15) | (((byte(8 + (is & 3)) >> (2 * (is >> 2))) & 3) << 4)) - 32;
 }
 template <> struct Raw<Q3_K> {
-    static constexpr bool mins = false, g16 = true, per_chunk = false;
+    static constexpr bool mins = false, g16 = true;
     uint2 qv[2], hm; uint32_t sc[3], d;
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         qv[0] = ld8_2a(blk + 32 + 8 * q);
@@ -264,33 +233,9 @@ template <> struct Raw<Q3_K> {
     }
     __device__ __forceinline__ float fold(int si, int) const { return h2f(d) * (float) si; }
 };
-// Q6_K (210 B): chunk c = elements 32 c ..: hf = c >> 2, qt = c & 3; lane values l = 8 q .. + 7 from
-// ql[64 hf + 32 (qt & 1) + l] (high nibble when qt >= 2) and bits 2 qt of qh[32 hf + l]; groups 2 c, 2 c + 1.
-template <> struct Raw<Q6_K> {
-    static constexpr bool mins = false, g16 = true, per_chunk = false;
-    uint2 ql[4], qh[2]; uint4 scv; uint32_t d;
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ql[i] = ld8_2a(blk + 64 * (i >> 1) + 32 * (i & 1) + 8 * q);   // reads up to blk + 132
-#pragma unroll
-        for (int i = 0; i < 2; ++i) qh[i] = ld8_2a(blk + 128 + 32 * i + 8 * q);                     // up to blk + 196
-        scv = ld16_2a_tail(blk + 192);                                                                // up to blk + 210
-        d = ld_u16(blk + 208);
-    }
-    __device__ __forceinline__ void chunk(int c, int, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int hf = c >> 2, qt = c & 3, sh = qt >= 2 ? 4 : 0;
-        const uint2 l = ql[2 * hf + (qt & 1)], h = qh[hf];
-        b0 = q6_signed(((l.x >> sh) & 0x0F0F0F0Fu) | (((h.x >> (2 * qt)) & 0x03030303u) << 4));
-        b1 = q6_signed(((l.y >> sh) & 0x0F0F0F0Fu) | (((h.y >> (2 * qt)) & 0x03030303u) << 4));
-        s0 = (int) (int8_t) byte_of(scv, 2 * c);
-        s1 = (int) (int8_t) byte_of(scv, 2 * c + 1);
-        mn = 0;
-    }
-    __device__ __forceinline__ float fold(int si, int) const { return h2f(d) * (float) si; }
-};
 // IQ4_XS (136 B): chunk c = 32-group c; lane values 8 q .. + 7 are nibbles (q >> 1) of qs[16 c + 8 (q & 1) ..]
 template <> struct Raw<IQ4_XS> {
-    static constexpr bool mins = false, g16 = false, per_chunk = false;
+    static constexpr bool mins = false, g16 = false;
     uint2 qv[8]; uint32_t dsh, sl;
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -307,36 +252,11 @@ template <> struct Raw<IQ4_XS> {
     }
     __device__ __forceinline__ float fold(int si, int) const { return h2f(dsh & 0xffff) * (float) si; }
 };
-// IQ2_XS (74 B): chunk c = 32-group c; lane q takes 8-group q (grid row qs[4 c + q], signs); scales
-// 2 (scales[c] & 15) + 1 for k 0..15 (lanes q < 2) and 2 (scales[c] >> 4) + 1 for k 16..31.
-template <> struct Raw<IQ2_XS> {
-    static constexpr bool mins = false, g16 = true, per_chunk = false;
-    uint32_t qq[4]; uint2 scv; uint32_t d;
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-#pragma unroll
-        for (int c = 0; c < 8; c += 2) qq[c >> 1] = (uint32_t) ld_u16(blk + 2 + 2 * (4 * c + q)) | ((uint32_t) ld_u16(blk + 2 + 2 * (4 * c + 4 + q)) << 16);
-        scv = make_uint2((uint32_t) ld_u16(blk + 66) | ((uint32_t) ld_u16(blk + 68) << 16),
-                         (uint32_t) ld_u16(blk + 70) | ((uint32_t) ld_u16(blk + 72) << 16));
-        d = ld_u16(blk);
-    }
-    __device__ __forceinline__ void chunk(int c, int, const uint2 *grid, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const uint32_t qv = (qq[c >> 1] >> (16 * (c & 1))) & 0xffff;
-        const uint2 g = grid[qv & 511], sm = grid[512 + (qv >> 9)];
-        b0 = apply_mask(g.x, sm.x);
-        b1 = apply_mask(g.y, sm.y);
-        const uint32_t s = ((c < 4 ? scv.x : scv.y) >> (8 * (c & 3))) & 0xff;
-        s0 = 2 * (int) (s & 15) + 1;
-        s1 = 2 * (int) (s >> 4) + 1;
-        mn = 0;
-    }
-    __device__ __forceinline__ float fold(int si, int) const { return (h2f(d) * 0.125f) * (float) si; }
-};
-
 // IQ2_XXS (66 B): chunk c = 32-group c, two words at 2 + 8 c (grid rows a byte each, then 4 x 7 sign bits and the
 // 4-bit scale); lane q takes 8-group q: grid row byte q of the first word, signs bits 7 q .. of the second, the chunk's
 // scale 2 sc + 1 (src/kernels4.cu:578-589; ggml's vec_dot_iq2_xxs_q8_K integers).
 template <> struct Raw<IQ2_XXS> {
-    static constexpr bool mins = false, g16 = false, per_chunk = false;
+    static constexpr bool mins = false, g16 = false;
     uint32_t gi[2], a1[8], d;   // gi: the lane's grid row of chunk c in byte c % 4 of gi[c / 4]
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         gi[0] = gi[1] = 0;
@@ -361,7 +281,7 @@ template <> struct Raw<IQ2_XXS> {
 // IQ4_NL (8 blocks of 18 B per 256 values, Q8_0 activations): chunk c = block c; lane values 8 q .. + 7 are
 // nibbles (q >> 1) of qs[8 (q & 1) ..]; every block folds on its own: acc = fma(x_d, fp16(d_c) * D, acc).
 template <> struct Raw<IQ4_NL> {
-    static constexpr bool mins = false, g16 = false, per_chunk = true;
+    static constexpr bool mins = false, g16 = false;
     uint2 qv[8]; uint32_t dd[4];
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
         // the span is 16-byte aligned (rows of 144 n / 256 bytes), so block c's qs sit at 2 mod 4 for even c and
@@ -393,7 +313,7 @@ template <> struct Raw<IQ4_NL> {
 // so block c's qs (34 c + 2) are 2 mod 4 for even c, read by ld8_2a whose 12 bytes end at most at blk + 239, and
 // dword-aligned for odd c, read as they are: block 7's last 8 bytes end the span, and of the last row the allocation.
 template <> struct Raw<Q8_0> {
-    static constexpr bool mins = false, g16 = false, per_chunk = true;
+    static constexpr bool mins = false, g16 = false;
     uint2 qv[8]; uint32_t dd[4];
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -416,7 +336,7 @@ template <> struct Raw<Q8_0> {
 // aligned, so block c's qs at 17 c + 1 sit at offset (17 c + 1) mod 4 = 1 2 3 0 1 2 3 0: the dword-aligned ones
 // (c = 3, 7) are read as they are, the others by ld8_2a, whose 12 bytes end at most at blk + 119.
 template <> struct Raw<MXFP4> {
-    static constexpr bool mins = false, g16 = false, per_chunk = true;
+    static constexpr bool mins = false, g16 = false;
     uint2 qv[8]; uint32_t ee[2];
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -442,7 +362,7 @@ template <> struct Raw<MXFP4> {
 // span).  The min's term needs each token's block sum q: chunk_fold takes it from one more MFMA against ones
 // (ysum), and the fold is fma(d_c, D, m_c * S) (the integers of Item<Q5_1>).
 template <> struct Raw<Q5_1> {
-    static constexpr bool mins = false, g16 = false, per_chunk = true;
+    static constexpr bool mins = false, g16 = false;
     uint2 qv[8]; uint32_t hb[2], dm[8];
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -472,7 +392,7 @@ template <> struct Raw<Q5_1> {
 // where the bit is clear (x - 16 as int8).  Block c's qs (22 c + 6) and qh (22 c + 2) are 2 mod 4 for even c, read by
 // ld8_2a whose 12 bytes end at most at blk + 155, and dword-aligned for odd c, read as they are.
 template <> struct Raw<Q5_0> {
-    static constexpr bool mins = false, g16 = false, per_chunk = true;
+    static constexpr bool mins = false, g16 = false;
     uint2 qv[8]; uint32_t hb[2], dd[4];
     __device__ __forceinline__ void load(const uint8_t *blk, int q) {
 #pragma unroll
@@ -588,7 +508,7 @@ __device__ __forceinline__ int mul_bytes(uint32_t q, uint32_t f) {
 // (chunk 2j + 1) for q >= 2.  Every lane's 16 values lie in one chunk, so its 6-bit scale s = 8 a + b (a, b < 8) is
 // applied inside B: D1 = sum a_c dot_c and D2 = sum b_c dot_c (a q, b q < 128 fit int8), sum_c s_c dot_c = 8 D1 + D2
 // exactly; a third MFMA against the chunk mins gives sum_c m_c sum(x_c).
-// Token tiles T0 .. T0 + NT - 1 (compile-time: straight-line code, accumulators only for the tiles present)
+// Token tiles 0 .. NT - 1 (compile-time: straight-line code, accumulators only for the tiles present)
 // The lane's constants (quarter, row, offsets, selectors) are derived in the step from a lane id the compiler cannot
 // hoist: recomputing them costs a few instructions, keeping them live across the stream would cost registers.
 __device__ __forceinline__ int lane_id_here() {
@@ -596,12 +516,12 @@ __device__ __forceinline__ int lane_id_here() {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
     return l;
 }
-template <int NT, int T0, bool FIRST>
+template <int NT, bool FIRST>
 __device__ __forceinline__ void step_q4k(const uint8_t *wl0, const int8_t *as, const float *yd, float (&acc)[GM_TILES][4]) {
     // the tiles past NT hold nothing this item reads (a tile count is fixed for an item, and an item's first span
     // writes its tiles without reading them): marking them redefined frees their registers in this step
 #pragma unroll
-    for (int t = T0 + NT; t < GM_TILES; ++t)
+    for (int t = NT; t < GM_TILES; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
     const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
@@ -630,7 +550,7 @@ __device__ __forceinline__ void step_q4k(const uint8_t *wl0, const int8_t *as, c
         const uint32_t aj = a0 ^ (64 * j);   // piece 4 j + q
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const v4i A = lds_at<v4i>(aj + (T0 + t) * 16 * 256);
+            const v4i A = lds_at<v4i>(aj + t * 16 * 256);
             d1[t] = mfma64(A, B1, j ? d1[t] : z);
             d2[t] = mfma64(A, B2, j ? d2[t] : z);
             dm[t] = mfma64(A, Bm, j ? dm[t] : z);
@@ -643,7 +563,7 @@ __device__ __forceinline__ void step_q4k(const uint8_t *wl0, const int8_t *as, c
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int si = (d1[t][v] << 3) + d2[t][v];
-            acc[T0 + t][v] = __builtin_fmaf(yd[(T0 + t) * 16 + 4 * q + v], __builtin_fmaf(d, (float) si, -(dmin * (float) dm[t][v])), FIRST ? 0.0f : acc[T0 + t][v]);
+            acc[t][v] = __builtin_fmaf(yd[t * 16 + 4 * q + v], __builtin_fmaf(d, (float) si, -(dmin * (float) dm[t][v])), FIRST ? 0.0f : acc[t][v]);
         }
     }
 }
@@ -664,12 +584,12 @@ typedef short v2i16 __attribute__((ext_vector_type(2)));
 // [-64, 64], L = B & 63): D_H = X.H and D_L = X.L give sum_g sc_g dot_g = 64 D_H + D_L exactly.  The lane's values sit
 // in ql[64 (j / 2) + 16 q ..] (nibble j % 2) and qh[32 (j / 2) + 16 (q % 2) ..] (bits 4 (j % 2) + 2 (q / 2)); rows of
 // the 210-byte blocks are 2-byte aligned in LDS, so 16-byte reads go through ld16_u2.
-template <int NT, int T0, bool FIRST>
+template <int NT, bool FIRST>
 __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, const float *yd, float (&acc)[GM_TILES][4]) {
     // the tiles past NT hold nothing this item reads (a tile count is fixed for an item, and an item's first span
     // writes its tiles without reading them): marking them redefined frees their registers in this step
 #pragma unroll
-    for (int t = T0 + NT; t < GM_TILES; ++t)
+    for (int t = NT; t < GM_TILES; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
     const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
@@ -711,7 +631,7 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
         const uint32_t aj = a0 ^ (64 * j);   // piece 4 j + q
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const v4i A = lds_at<v4i>(aj + (T0 + t) * 16 * 256);
+            const v4i A = lds_at<v4i>(aj + t * 16 * 256);
             dh[t] = mfma64(A, Bh, j ? dh[t] : z);
             dl[t] = mfma64(A, Bl, j ? dl[t] : z);
             asm volatile("");   // a scheduling-region boundary: operands are not hoisted across tiles (register pressure)
@@ -722,7 +642,7 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int si = (dh[t][v] << 6) + dl[t][v];
-            acc[T0 + t][v] = __builtin_fmaf(yd[(T0 + t) * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[T0 + t][v]);
+            acc[t][v] = __builtin_fmaf(yd[t * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[t][v]);
         }
     }
     asm volatile("");   // keeps the tile-count variants from being merged (which moved the accumulators to memory)
@@ -771,11 +691,11 @@ __device__ __forceinline__ uint32_t ld4_u2(const uint8_t *p, uint32_t sb) {
     const uint32_t *w = (const uint32_t *) (p - sb);
     return __builtin_amdgcn_alignbyte(w[1], w[0], sb);
 }
-template <int NT, int T0, bool FIRST>
+template <int NT, bool FIRST>
 __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as, const float *yd, const uint32_t *sel, float (&acc)[GM_TILES][4]) {
     // the tiles past NT hold nothing this item reads: marking them redefined frees their registers (as in step_q4k)
 #pragma unroll
-    for (int t = T0 + NT; t < GM_TILES; ++t)
+    for (int t = NT; t < GM_TILES; ++t)
 #pragma unroll
         for (int v = 0; v < 4; ++v) asm volatile("" : "=v"(acc[t][v]));
     const int lid = lane_id_here(), q = lid >> 4, rr = lid & 15;
@@ -812,7 +732,7 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
         const uint32_t aj = a0 ^ (64 * j);   // piece 4 j + q
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const v4i A = lds_at<v4i>(aj + (T0 + t) * 16 * 256);
+            const v4i A = lds_at<v4i>(aj + t * 16 * 256);
             dp[t] = mfma64(A, BP, j ? dp[t] : z);
             dq[t] = mfma64(A, BQ, j ? dq[t] : z);
             asm volatile("");   // a scheduling-region boundary: operands are not hoisted across tiles (register pressure)
@@ -823,7 +743,7 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int si = (dp[t][v] << 4) + dq[t][v];
-            acc[T0 + t][v] = __builtin_fmaf(yd[(T0 + t) * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[T0 + t][v]);
+            acc[t][v] = __builtin_fmaf(yd[t * 16 + 4 * q + v], d * (float) si, FIRST ? 0.0f : acc[t][v]);
         }
     }
     asm volatile("");   // keeps the tile-count variants from being merged
@@ -1339,34 +1259,34 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                 // after the epilogue, so the accumulators stay in the same registers on every path through the loop
                 if (b == 0) {
                     switch (ntile) {
-                    case 1: step_q4k<1, 0, true>(wt, as, yd, acc); break;
-                    case 2: step_q4k<2, 0, true>(wt, as, yd, acc); break;
-                    case 3: step_q4k<3, 0, true>(wt, as, yd, acc); break;
-                    default: step_q4k<4, 0, true>(wt, as, yd, acc); break;
+                    case 1: step_q4k<1, true>(wt, as, yd, acc); break;
+                    case 2: step_q4k<2, true>(wt, as, yd, acc); break;
+                    case 3: step_q4k<3, true>(wt, as, yd, acc); break;
+                    default: step_q4k<4, true>(wt, as, yd, acc); break;
                     }
                 } else {
                     switch (ntile) {
-                    case 1: step_q4k<1, 0, false>(wt, as, yd, acc); break;
-                    case 2: step_q4k<2, 0, false>(wt, as, yd, acc); break;
-                    case 3: step_q4k<3, 0, false>(wt, as, yd, acc); break;
-                    default: step_q4k<4, 0, false>(wt, as, yd, acc); break;
+                    case 1: step_q4k<1, false>(wt, as, yd, acc); break;
+                    case 2: step_q4k<2, false>(wt, as, yd, acc); break;
+                    case 3: step_q4k<3, false>(wt, as, yd, acc); break;
+                    default: step_q4k<4, false>(wt, as, yd, acc); break;
                     }
                 }
             } else if constexpr (T == Q6_K) {
                 const uint8_t *wt = stage_w(stage) + wave * C::TB;
                 if (b == 0) {
                     switch (ntile) {
-                    case 1: step_q6k<1, 0, true>(wt, as, yd, acc); break;
-                    case 2: step_q6k<2, 0, true>(wt, as, yd, acc); break;
-                    case 3: step_q6k<3, 0, true>(wt, as, yd, acc); break;
-                    default: step_q6k<4, 0, true>(wt, as, yd, acc); break;
+                    case 1: step_q6k<1, true>(wt, as, yd, acc); break;
+                    case 2: step_q6k<2, true>(wt, as, yd, acc); break;
+                    case 3: step_q6k<3, true>(wt, as, yd, acc); break;
+                    default: step_q6k<4, true>(wt, as, yd, acc); break;
                     }
                 } else {
                     switch (ntile) {
-                    case 1: step_q6k<1, 0, false>(wt, as, yd, acc); break;
-                    case 2: step_q6k<2, 0, false>(wt, as, yd, acc); break;
-                    case 3: step_q6k<3, 0, false>(wt, as, yd, acc); break;
-                    default: step_q6k<4, 0, false>(wt, as, yd, acc); break;
+                    case 1: step_q6k<1, false>(wt, as, yd, acc); break;
+                    case 2: step_q6k<2, false>(wt, as, yd, acc); break;
+                    case 3: step_q6k<3, false>(wt, as, yd, acc); break;
+                    default: step_q6k<4, false>(wt, as, yd, acc); break;
                     }
                 }
             } else if constexpr (T == IQ2_XS) {
@@ -1374,35 +1294,34 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
                 const uint32_t *sel = (const uint32_t *) smem;
                 if (b == 0) {
                     switch (ntile) {
-                    case 1: step_iq2xs<1, 0, true>(wt, as, yd, sel, acc); break;
-                    case 2: step_iq2xs<2, 0, true>(wt, as, yd, sel, acc); break;
-                    case 3: step_iq2xs<3, 0, true>(wt, as, yd, sel, acc); break;
-                    default: step_iq2xs<4, 0, true>(wt, as, yd, sel, acc); break;
+                    case 1: step_iq2xs<1, true>(wt, as, yd, sel, acc); break;
+                    case 2: step_iq2xs<2, true>(wt, as, yd, sel, acc); break;
+                    case 3: step_iq2xs<3, true>(wt, as, yd, sel, acc); break;
+                    default: step_iq2xs<4, true>(wt, as, yd, sel, acc); break;
                     }
                 } else {
                     switch (ntile) {
-                    case 1: step_iq2xs<1, 0, false>(wt, as, yd, sel, acc); break;
-                    case 2: step_iq2xs<2, 0, false>(wt, as, yd, sel, acc); break;
-                    case 3: step_iq2xs<3, 0, false>(wt, as, yd, sel, acc); break;
-                    default: step_iq2xs<4, 0, false>(wt, as, yd, sel, acc); break;
+                    case 1: step_iq2xs<1, false>(wt, as, yd, sel, acc); break;
+                    case 2: step_iq2xs<2, false>(wt, as, yd, sel, acc); break;
+                    case 3: step_iq2xs<3, false>(wt, as, yd, sel, acc); break;
+                    default: step_iq2xs<4, false>(wt, as, yd, sel, acc); break;
                     }
                 }
             } else {
                 const uint8_t *wt = stage_w(stage) + wave * C::TB;
-                constexpr int TT = A0 ? (int) Q4_K : T;   // (the A0 types never come here)
                 if (b == 0) {
                     switch (ntile) {
-                    case 1: step_gen<TT, 1, true>(wt, grid, as, yd, acc); break;
-                    case 2: step_gen<TT, 2, true>(wt, grid, as, yd, acc); break;
-                    case 3: step_gen<TT, 3, true>(wt, grid, as, yd, acc); break;
-                    default: step_gen<TT, 4, true>(wt, grid, as, yd, acc); break;
+                    case 1: step_gen<T, 1, true>(wt, grid, as, yd, acc); break;
+                    case 2: step_gen<T, 2, true>(wt, grid, as, yd, acc); break;
+                    case 3: step_gen<T, 3, true>(wt, grid, as, yd, acc); break;
+                    default: step_gen<T, 4, true>(wt, grid, as, yd, acc); break;
                     }
                 } else {
                     switch (ntile) {
-                    case 1: step_gen<TT, 1, false>(wt, grid, as, yd, acc); break;
-                    case 2: step_gen<TT, 2, false>(wt, grid, as, yd, acc); break;
-                    case 3: step_gen<TT, 3, false>(wt, grid, as, yd, acc); break;
-                    default: step_gen<TT, 4, false>(wt, grid, as, yd, acc); break;
+                    case 1: step_gen<T, 1, false>(wt, grid, as, yd, acc); break;
+                    case 2: step_gen<T, 2, false>(wt, grid, as, yd, acc); break;
+                    case 3: step_gen<T, 3, false>(wt, grid, as, yd, acc); break;
+                    default: step_gen<T, 4, false>(wt, grid, as, yd, acc); break;
                     }
                 }
             }
