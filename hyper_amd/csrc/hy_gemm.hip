@@ -25,19 +25,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ v4i mfma16(long a, long b, v4i c) { return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, c, 0, 0, 0); }
 __device__ __forceinline__ long mk_long(uint32_t lo, uint32_t hi) { return (long) (((unsigned long long) hi << 32) | lo); }
-
-// Branch-free loads from 2-byte aligned addresses (a fixed instruction count per step lets the compiler count
-// the loads in flight): whole dwords from the aligned-down address, joined with v_alignbyte.
-__device__ __forceinline__ uint32_t join_b(uint32_t hi, uint32_t lo, uint32_t sb) { return __builtin_amdgcn_alignbyte(hi, lo, sb); }
-// 8 bytes at p (2-byte aligned); reads the dwords at p & ~3 .. + 11, all of which must lie in the buffer
-// (the aligned-down pointer is formed by pointer arithmetic on p, so that an LDS pointer stays an LDS pointer)
-__device__ __forceinline__ uint2 ld8_2a(const uint8_t *p) {
-    const uint32_t *w = (const uint32_t *) (p - ((uintptr_t) p & 3));
-    const uint32_t sb = (uint32_t) ((uintptr_t) p & 3);
-    const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
-    return make_uint2(join_b(d1, d0, sb), join_b(d2, d1, sb));
-}
-
 // The raw bytes of one weight row's 256-value block that lane quarter q needs, and their decoding per 32-value
 // chunk c: B operand words b0/b1 (8 int8 values), scale(s), min.
 template <int T> struct Raw;
@@ -276,145 +263,6 @@ template <> struct Raw<IQ2_XXS> {
         s1 = 0; mn = 0;
     }
     __device__ __forceinline__ float fold(int si, int) const { return (h2f(d) * 0.125f) * (float) si; }
-};
-
-// IQ4_NL (8 blocks of 18 B per 256 values, Q8_0 activations): chunk c = block c; lane values 8 q .. + 7 are
-// nibbles (q >> 1) of qs[8 (q & 1) ..]; every block folds on its own: acc = fma(x_d, fp16(d_c) * D, acc).
-template <> struct Raw<IQ4_NL> {
-    static constexpr bool mins = false, g16 = false;
-    uint2 qv[8]; uint32_t dd[4];
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-        // the span is 16-byte aligned (rows of 144 n / 256 bytes), so block c's qs sit at 2 mod 4 for even c and
-        // at 0 mod 4 for odd c
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint8_t *p = blk + 18 * c + 2 + 8 * (q & 1);
-            if (c & 1) qv[c] = *(const uint2 *) p;
-            else {
-                const uint32_t *w = (const uint32_t *) (p - 2);
-                const uint32_t d0 = w[0], d1 = w[1], d2 = w[2];
-                qv[c] = make_uint2(join_b(d1, d0, 2), join_b(d2, d1, 2));
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dd[i] = (uint32_t) ld_u16(blk + 36 * i) | ((uint32_t) ld_u16(blk + 36 * i + 18) << 16);
-    }
-    __device__ __forceinline__ void chunk(int c, int q, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int s = 4 * (q >> 1);
-        b0 = kv4((qv[c].x >> s) & 0x0F0F0F0Fu);
-        b1 = kv4((qv[c].y >> s) & 0x0F0F0F0Fu);
-        s0 = 1; s1 = 0; mn = 0;
-    }
-    __device__ __forceinline__ float cfold(int c, int d) const { return h2f((dd[c >> 1] >> (16 * (c & 1))) & 0xffff) * (float) d; }
-    __device__ __forceinline__ float fold(int si, int) const { return (float) si; }
-};
-// Q8_0 weights (8 blocks of 34 B per 256 values, Q8_0 activations): chunk c = block c; lane values 8 q .. + 7 are
-// qs[8 q ..] of block c as they are (int8); every block folds on its own, as IQ4_NL's.  The spans are 16-byte aligned,
-// so block c's qs (34 c + 2) are 2 mod 4 for even c, read by ld8_2a whose 12 bytes end at most at blk + 239, and
-// dword-aligned for odd c, read as they are: block 7's last 8 bytes end the span, and of the last row the allocation.
-template <> struct Raw<Q8_0> {
-    static constexpr bool mins = false, g16 = false;
-    uint2 qv[8]; uint32_t dd[4];
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint8_t *p = blk + 34 * c + 2 + 8 * q;
-            qv[c] = (c & 1) ? *(const uint2 *) p : ld8_2a(p);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dd[i] = (uint32_t) ld_u16(blk + 68 * i) | ((uint32_t) ld_u16(blk + 68 * i + 34) << 16);
-    }
-    __device__ __forceinline__ void chunk(int c, int, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        b0 = qv[c].x; b1 = qv[c].y;
-        s0 = 1; s1 = 0; mn = 0;
-    }
-    __device__ __forceinline__ float cfold(int c, int d) const { return h2f((dd[c >> 1] >> (16 * (c & 1))) & 0xffff) * (float) d; }
-    __device__ __forceinline__ float fold(int si, int) const { return (float) si; }
-};
-// MXFP4 (8 blocks of 17 B per 256 values, Q8_0 activations): chunk c = block c, lane values as IQ4_NL's (nibbles
-// (q >> 1) of qs[8 (q & 1) ..]), the MXFP4 codebook, the fold e8m0_half(e_c) * D.  Spans of 136 bytes are 8-byte
-// aligned, so block c's qs at 17 c + 1 sit at offset (17 c + 1) mod 4 = 1 2 3 0 1 2 3 0: the dword-aligned ones
-// (c = 3, 7) are read as they are, the others by ld8_2a, whose 12 bytes end at most at blk + 119.
-template <> struct Raw<MXFP4> {
-    static constexpr bool mins = false, g16 = false;
-    uint2 qv[8]; uint32_t ee[2];
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint8_t *p = blk + 17 * c + 1 + 8 * (q & 1);
-            qv[c] = (c & 3) == 3 ? *(const uint2 *) p : ld8_2a(p);
-        }
-        ee[0] = ee[1] = 0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) ee[c >> 2] |= (uint32_t) blk[17 * c] << (8 * (c & 3));
-    }
-    __device__ __forceinline__ void chunk(int c, int q, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int s = 4 * (q >> 1);
-        b0 = kvfp4((qv[c].x >> s) & 0x0F0F0F0Fu);
-        b1 = kvfp4((qv[c].y >> s) & 0x0F0F0F0Fu);
-        s0 = 1; s1 = 0; mn = 0;
-    }
-    __device__ __forceinline__ float cfold(int c, int d) const { return e8m0_half((ee[c >> 2] >> (8 * (c & 3))) & 255) * (float) d; }
-    __device__ __forceinline__ float fold(int si, int) const { return (float) si; }
-};
-// Q5_1 (8 blocks of 24 B per 256 values, Q8_0 activations): chunk c = block c, lane values as IQ4_NL's with the fifth
-// bits in qh byte q of the block (x = nibble | bit << 4, 0..31); every field dword-aligned (24-byte blocks in a 192-byte
-// span).  The min's term needs each token's block sum q: chunk_fold takes it from one more MFMA against ones
-// (ysum), and the fold is fma(d_c, D, m_c * S) (the integers of Item<Q5_1>).
-template <> struct Raw<Q5_1> {
-    static constexpr bool mins = false, g16 = false;
-    uint2 qv[8]; uint32_t hb[2], dm[8];
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            qv[c] = *(const uint2 *) (blk + 24 * c + 8 + 8 * (q & 1));
-            dm[c] = *(const uint32_t *) (blk + 24 * c);
-        }
-        hb[0] = hb[1] = 0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) hb[c >> 2] |= (uint32_t) blk[24 * c + 4 + q] << (8 * (c & 3));
-    }
-    __device__ __forceinline__ void chunk(int c, int q, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int s = 4 * (q >> 1);
-        const uint32_t h = hb[c >> 2] >> (8 * (c & 3));
-        b0 = ((qv[c].x >> s) & 0x0F0F0F0Fu) | (spread4(h & 15) << 4);
-        b1 = ((qv[c].y >> s) & 0x0F0F0F0Fu) | (spread4((h >> 4) & 15) << 4);
-        s0 = 1; s1 = 0; mn = 0;
-    }
-    __device__ __forceinline__ float cfold2(int c, int d, int ys) const {
-        return __builtin_fmaf(h2f(dm[c] & 0xffff), (float) d, h2f(dm[c] >> 16) * (float) ys);
-    }
-    __device__ __forceinline__ float cfold(int c, int d) const { return cfold2(c, d, 0); }
-    __device__ __forceinline__ float fold(int si, int) const { return (float) si; }
-};
-// Q5_0 (8 blocks of 22 B per 256 values, Q8_0 activations): chunk c = block c, lane values as IQ4_NL's (nibbles
-// (q >> 1) of qs[8 (q & 1) ..]) with their fifth bits in qh byte q (bits 8 q .. 8 q + 7), each byte nibble | 0xF0
-// where the bit is clear (x - 16 as int8).  Block c's qs (22 c + 6) and qh (22 c + 2) are 2 mod 4 for even c, read by
-// ld8_2a whose 12 bytes end at most at blk + 155, and dword-aligned for odd c, read as they are.
-template <> struct Raw<Q5_0> {
-    static constexpr bool mins = false, g16 = false;
-    uint2 qv[8]; uint32_t hb[2], dd[4];
-    __device__ __forceinline__ void load(const uint8_t *blk, int q) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint8_t *p = blk + 22 * c + 6 + 8 * (q & 1);
-            qv[c] = (c & 1) ? *(const uint2 *) p : ld8_2a(p);
-        }
-        hb[0] = hb[1] = 0;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) hb[c >> 2] |= (uint32_t) blk[22 * c + 2 + q] << (8 * (c & 3));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dd[i] = (uint32_t) ld_u16(blk + 44 * i) | ((uint32_t) ld_u16(blk + 44 * i + 22) << 16);
-    }
-    __device__ __forceinline__ void chunk(int c, int q, const uint2 *, uint32_t &b0, uint32_t &b1, int &s0, int &s1, int &mn) const {
-        const int s = 4 * (q >> 1);
-        const uint32_t nh = ~(hb[c >> 2] >> (8 * (c & 3)));
-        b0 = ((qv[c].x >> s) & 0x0F0F0F0Fu) | fill_f0(nh & 15);
-        b1 = ((qv[c].y >> s) & 0x0F0F0F0Fu) | fill_f0((nh >> 4) & 15);
-        s0 = 1; s1 = 0; mn = 0;
-    }
-    __device__ __forceinline__ float cfold(int c, int d) const { return h2f((dd[c >> 1] >> (16 * (c & 1))) & 0xffff) * (float) d; }
-    __device__ __forceinline__ float fold(int si, int) const { return (float) si; }
 };
 
 constexpr int GM_TOK = 64, GM_TILES = GM_TOK / 16, GM_ROWS = 64, GM_LD = 264;   // LDS row stride of staged activations
@@ -1428,27 +1276,61 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     }
 }
 
-// IQ4_NL / Q8_0 / MXFP4 / Q5_0 / Q5_1: one chunk's MFMA per tile folded straight into the fp32 accumulators (Yc: 8 block scales per token)
+// A lane's bytes of a span (SpanBytes) as its B words of 32-value block c -- values 8 q .. + 7 -- and the block's fold of the
+// exact integer d (and, Q5_1, the token block's sum of quants s).
+template <int T> struct Staged;
+template <> struct Staged<IQ4_NL> : SpanBytes<IQ4_NL> {
+    __device__ __forceinline__ long b(int c, int q) const {
+        const int s = 4 * (q >> 1);
+        return mk_long(kv4((qv[c].x >> s) & 0x0F0F0F0Fu), kv4((qv[c].y >> s) & 0x0F0F0F0Fu));
+    }
+    __device__ __forceinline__ float fold(int c, int d, int) const { return h2f((dd[c >> 1] >> (16 * (c & 1))) & 0xffff) * (float) d; }
+};
+template <> struct Staged<Q8_0> : SpanBytes<Q8_0> {
+    __device__ __forceinline__ long b(int c, int) const { return mk_long(qv[c].x, qv[c].y); }
+    __device__ __forceinline__ float fold(int c, int d, int) const { return h2f((dd[c >> 1] >> (16 * (c & 1))) & 0xffff) * (float) d; }
+};
+template <> struct Staged<MXFP4> : SpanBytes<MXFP4> {
+    __device__ __forceinline__ long b(int c, int q) const {
+        const int s = 4 * (q >> 1);
+        return mk_long(kvfp4((qv[c].x >> s) & 0x0F0F0F0Fu), kvfp4((qv[c].y >> s) & 0x0F0F0F0Fu));
+    }
+    __device__ __forceinline__ float fold(int c, int d, int) const { return e8m0_half((ee[c >> 2] >> (8 * (c & 3))) & 255) * (float) d; }
+};
+template <> struct Staged<Q5_1> : SpanBytes<Q5_1> {   // x = nibble | bit << 4, 0..31
+    __device__ __forceinline__ long b(int c, int q) const {
+        const int s = 4 * (q >> 1);
+        const uint32_t h = hb[c >> 2] >> (8 * (c & 3));
+        return mk_long(((qv[c].x >> s) & 0x0F0F0F0Fu) | (spread4(h & 15) << 4), ((qv[c].y >> s) & 0x0F0F0F0Fu) | (spread4((h >> 4) & 15) << 4));
+    }
+    __device__ __forceinline__ float fold(int c, int d, int s) const {
+        return __builtin_fmaf(h2f(dm[c] & 0xffff), (float) d, h2f(dm[c] >> 16) * (float) s);
+    }
+};
+template <> struct Staged<Q5_0> : SpanBytes<Q5_0> {   // each byte nibble | 0xF0 where the fifth bit is clear (x - 16 as int8)
+    __device__ __forceinline__ long b(int c, int q) const {
+        const int s = 4 * (q >> 1);
+        const uint32_t nh = ~(hb[c >> 2] >> (8 * (c & 3)));
+        return mk_long(((qv[c].x >> s) & 0x0F0F0F0Fu) | fill_f0(nh & 15), ((qv[c].y >> s) & 0x0F0F0F0Fu) | fill_f0((nh >> 4) & 15));
+    }
+    __device__ __forceinline__ float fold(int c, int d, int) const { return h2f((dd[c >> 1] >> (16 * (c & 1))) & 0xffff) * (float) d; }
+};
+
+// one block's MFMA per tile, folded straight into the fp32 accumulators (Yc: 8 block scales per token)
 template <int T>
-__device__ __forceinline__ void chunk_fold(const Raw<T> &w, int c, int q, const int8_t *As, const float *Yc, int rr, int ntile,
+__device__ __forceinline__ void chunk_fold(const Staged<T> &w, int c, int q, const int8_t *As, const float *Yc, int rr, int ntile,
                                            float (&acc)[GM_TILES][4]) {
     const v4i z = {0, 0, 0, 0};
-    uint32_t b0, b1;
-    int s0, s1, mn;
-    w.chunk(c, q, nullptr, b0, b1, s0, s1, mn);
+    const long b = w.b(c, q);
 #pragma unroll
     for (int tile = 0; tile < GM_TILES; ++tile) {
         if (tile >= ntile) break;
         const long a = *(const long *) (As + (tile * 16 + rr) * GM_LD + 32 * c + 8 * q);
-        const v4i d0 = mfma16(a, mk_long(b0, b1), z);
-        if constexpr (ysum_type(T)) {   // each token's block sum: the same A against ones
-            const v4i d1 = mfma16(a, mk_long(0x01010101u, 0x01010101u), z);
+        const v4i d = mfma16(a, b, z);
+        v4i s = z;
+        if constexpr (ysum_type(T)) s = mfma16(a, mk_long(0x01010101u, 0x01010101u), z);   // each token's block sum: A against ones
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[tile][v] = __builtin_fmaf(Yc[(tile * 16 + 4 * q + v) * 8 + c], w.cfold2(c, d0[v], d1[v]), acc[tile][v]);
-        } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[tile][v] = __builtin_fmaf(Yc[(tile * 16 + 4 * q + v) * 8 + c], w.cfold(c, d0[v]), acc[tile][v]);
-        }
+        for (int v = 0; v < 4; ++v) acc[tile][v] = __builtin_fmaf(Yc[(tile * 16 + 4 * q + v) * 8 + c], w.fold(c, d[v], s[v]), acc[tile][v]);
     }
 }
 
@@ -1535,7 +1417,7 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
     };
 
     ItemState cur = locate(it);
-    Raw<T> w;
+    Staged<T> w;
     w.load(cur.W, q);
     uint4 a[4];
     float yd[2];
@@ -1558,7 +1440,7 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
         const int nit = last_b ? it + (int) gridDim.y : it;
         const bool more = nit < total;
         ItemState nxt = cur;
-        Raw<T> nw;
+        Staged<T> nw;
         if (more) {
             if (last_b) nxt = locate(nit);
             const int nb = last_b ? 0 : b + 1;

@@ -1,5 +1,6 @@
-"""Grouped GEMMs whose expert matrices end an allocation exactly: the last expert's last block is the allocation's last
-bytes, so a read past a block's end leaves it."""
+"""Grouped GEMMs over many experts with expert matrices of whole 2 MiB pages, the last expert among the routed ones.  What
+the loads of a span may read is checked on the CPU (tests/test_sanitize.py): here a read past the end would show only where
+nothing is mapped behind the matrix."""
 import pytest
 import torch
 

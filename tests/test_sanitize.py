@@ -1,6 +1,7 @@
 """The CPU-side C code under AddressSanitizer and UBSan (host builds only, tests/sanitize/Makefile): the oracle on every
 entry point and weight type, and the GGUF reader on well-formed and 300 corrupted files (truncations and byte flips,
-as tests/test_gguf.py makes them).  A sanitizer report aborts the driver, which fails the test."""
+as tests/test_gguf.py makes them); and the grouped GEMM's loads of weight spans from global memory, compiled for the CPU,
+over tiles that end an allocation.  A sanitizer report aborts the driver, which fails the test."""
 import os
 import shutil
 import subprocess
@@ -33,6 +34,10 @@ def _run(exe, args, tmp_path):
 
 def test_oracle_under_asan_ubsan(built, tmp_path):
     assert "oracle_san: done" in _run(built / "oracle_san", [], tmp_path)
+
+
+def test_span_loads_stay_in_the_matrix(built, tmp_path):
+    assert "span_loads: 0 wrong" in _run(built / "span_loads", [], tmp_path)
 
 
 def test_gguf_reader_under_asan_ubsan(built, tmp_path):
