@@ -1509,7 +1509,7 @@ __global__ __launch_bounds__(256) void k_gemm_nl(hy_moe_dev m, const uint8_t *__
 // must stay below 2^16 (checked against the upper bound below, from the host)
 constexpr int GM_MAX_ITEMS = 1 << 16;
 // upper bound of the work items: sum over active experts of ceil(cnt / GM_TOK) <= ceil(P / GM_TOK) + active
-static int max_items(int n_pairs, int max_active) { return (n_pairs + GM_TOK - 1) / GM_TOK + max_active; }
+constexpr int max_items(int n_pairs, int max_active) { return (n_pairs + GM_TOK - 1) / GM_TOK + max_active; }
 // the current device's CU count (an attribute query: cheap, thread-safe, and right for each device)
 static int cu_count() {
     int dev = 0, cus = 0;
@@ -1538,11 +1538,15 @@ static int item_slots(int row_tiles, int n_pairs, int max_active, int per_cu, bo
     }
 // their waves a block: 16 where two weight stages of 256 rows leave room for the activation buffers, else 8
 constexpr int a0_waves(int t) { return 2 * 256 * span_bytes(t) + 4 * (GM_TOK * 8 * Q8_0_BYTES) <= 150 * 1024 ? 16 : 8; }
-// k_gemm's 32-bit activation offsets and 16-bit item counts hold (larger launches take k_gemm_nl)
-static bool a0_fits(int n_pairs, int k, int in_dim, int max_active) {
-    return (size_t) n_pairs * (in_dim / 256) * (8 * Q8_0_BYTES) < 0xFFFF0000u && (uint64_t) n_pairs * (uint64_t) k < (1ull << 32) &&
-           max_items(n_pairs, max_active) < GM_MAX_ITEMS;
+// k_gemm's 32-bit activation offsets, its pair / k by multiply-high and its 16-bit item counts hold (larger launches take
+// k_gemm_nl).  k: pairs a row of activations, so gate/up's offsets reach (n_pairs - 1) / k rows.
+constexpr bool a0_fits(int n_pairs, int k, int in_dim, int max_active) {
+    return (size_t) ((n_pairs - 1) / k + 1) * (in_dim / 256) * (8 * Q8_0_BYTES) < 0xFFFF0000u &&
+           (uint64_t) n_pairs * (uint64_t) k < (1ull << 32) && max_items(n_pairs, max_active) < GM_MAX_ITEMS;
 }
+static_assert(a0_fits(131072 * 8, 8, 28672, 1024), "4.0e9 bytes of activation rows, each of eight pairs");
+static_assert(!a0_fits(1024 * 1024, 1, 28672, 1024) && !a0_fits(142000 * 8, 8, 28672, 1024), "rows past 32-bit offsets");
+static_assert(!a0_fits(1 << 28, 64, 256, 1) && !a0_fits(64 * 65536, 8, 256, 1), "pairs past the multiply-high; items past 16 bits");
 
 // One k_gemm launch: W waves a block, B blocks a CU (8 W output rows a block for gate/up, 16 W for down; ff and n are
 // multiples of 256, so 8 and 16 waves both tile them).
