@@ -395,7 +395,7 @@ int hy_moe_gate_up_q8(const hy_moe_dev *m, const void *xq, const int32_t *ids, i
     if (rc) return rc;
     if (!xq || !ids || !h || k <= 0 || nt < 0) { set_error("hy_moe_gate_up_q8: bad argument"); return HY_EINVAL; }
     if (n_expert <= 0 || n_expert > m->n_expert) { set_error("hy_moe_gate_up_q8: n_expert %d out of range", n_expert); return HY_EBAD_SHAPE; }
-    if ((uintptr_t) xq & 3) { set_error("hy_moe_gate_up_q8: xq must be 4-byte aligned"); return HY_EBAD_SHAPE; }
+    if (((uintptr_t) xq & 3) || !aligned16(hq)) { set_error("hy_moe_gate_up_q8: xq must be 4-byte and hq 16-byte aligned"); return HY_EBAD_SHAPE; }
     return launch_gate_up_ids(*m, xq, ids, n_expert, k, h, nt, s, (uint8_t *) hq);
 }
 

@@ -184,11 +184,19 @@ inline void moe_route_gate_up(const MoeDev &m, const float *logits, int ls, int 
 inline void moe_shared_gate_up(const MoeDev &m, const void *xq, float *h, int nt, hipStream_t s) {
     check(hy_moe_shared_gate_up(&m, xq, h, nt, s));
 }
+// the shared expert's decode down (moe_down with every id 0, k = 1, weight 1)
+inline void moe_shared_down(const MoeDev &m, const float *h, float *y, int nt, hipStream_t s) {
+    check(hy_moe_shared_down(&m, h, y, nt, s));
+}
 // moe_route_gate_up that also writes the hidden rows as Q8_0 blocks, and the down + combine that reads them (down types
 // whose partner is Q8_0)
 inline void moe_route_gate_up_q8(const MoeDev &m, const float *logits, int ls, int n_expert, int k, const void *xq, int *ids, float *wts,
                                  float *sg, float *h, void *hq, int nt, hipStream_t s) {
     check(hy_moe_route_gate_up_q8(&m, logits, ls, n_expert, k, xq, ids, wts, sg, h, hq, nt, s));
+}
+// moe_gate_up of pairs routed beforehand, from the Q8 rows of x; with hq also the Q8_0 hidden rows of moe_route_gate_up_q8
+inline void moe_gate_up_q8(const MoeDev &m, const void *xq, const int *ids, int n_expert, int k, float *h, void *hq, int nt, hipStream_t s) {
+    check(hy_moe_gate_up_q8(&m, xq, ids, n_expert, k, h, hq, nt, s));
 }
 inline void moe_down_reduce_q8(const MoeDev &m, const void *hq, const int *ids, const float *wts, int k, const float *shexp,
                                const float *sg, float *out, int residual, int nt, hipStream_t s) {

@@ -78,6 +78,12 @@ def test_cpp_header_compiles(tmp_path):
     assert r.returncode == 0, r.stderr
 
 
+def test_cpp_header_wraps_every_moe_entry():
+    text = (ROOT / "include/hymoe.hpp").read_text()
+    missing = [n for n in sorted(declared()) if n.startswith("hy_moe_") and not re.search(rf"check\({n}\(|return {n}\(", text)]
+    assert not missing, missing
+
+
 def test_tile_rows_layout():
     """tile_rows puts span s of row r at ((r // 16) * nspan + s) * 16 * sb + (r % 16) * sb of each expert, and the
     bytes of every span move whole."""
@@ -223,3 +229,28 @@ def test_n_local_is_required():
     assert b"n_local" in L.hy_last_error()
     assert L.hy_moe_order(ctypes.byref(m), p, 8, 128, p, p, None, p) == hyper_amd.HY_EINVAL
     assert L.hy_moe_down_reduce(ctypes.byref(m), p, p, p, 8, None, None, p, 1, None) == hyper_amd.HY_EINVAL
+
+
+def test_gate_up_q8_limits():
+    """hy_moe_gate_up_q8 refuses what its kernel does not hold before any launch, with the codes its header names."""
+    L = lib()
+    p = ctypes.c_void_p(16)
+
+    def call(m, E=128, k=8, hq=None, nt=1, xq=p):
+        return L.hy_moe_gate_up_q8(ctypes.byref(m), xq, p, E, k, p, hq, nt, None)
+
+    U, S, I = hyper_amd.HY_EUNSUPPORTED_TYPE, hyper_amd.HY_EBAD_SHAPE, hyper_amd.HY_EINVAL
+    assert call(_dev(n=8448)) == U                                # rows of more than 8192 values
+    assert call(_dev(E=1025), E=1025) == U
+    assert call(_dev(), nt=8192) == U                             # 65536 pairs
+    assert call(_dev(), E=129) == S and call(_dev(), E=0) == S    # ids past the slot table
+    assert call(_dev(), k=0) == I and call(_dev(), nt=-1) == I and call(_dev(), xq=None) == I
+    assert call(_dev(), xq=ctypes.c_void_p(18)) == S
+    assert call(_dev(), hq=p) == U                                # Q8_0 hidden rows of types with Q8_K rows
+    m = _dev()
+    m.tg = m.td = 8
+    m.gate_bytes = m.down_bytes = 768 * 2048 // 32 * 34
+    assert call(m, hq=ctypes.c_void_p(24)) == S                   # hq off a 16-byte boundary
+    m.n = 4352
+    m.gate_bytes = m.down_bytes = 768 * 4352 // 32 * 34
+    assert call(m, hq=p) == U                                     # Q8_0 hidden rows of n > 4096

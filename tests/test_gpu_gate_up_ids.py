@@ -1,5 +1,5 @@
 """Decode gate/up by ids from the Q8 rows (hy_moe_gate_up_q8): the bits of hy_moe_gate_up, with and without the Q8_0 hidden
-rows, absent experts left unwritten; its limits; a sigmoid-routed decode on it against the oracle."""
+rows, absent experts left unwritten; a sigmoid-routed decode on it, and past its limits, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -78,3 +78,32 @@ def test_sigmoid_decode(cuda, t, shared):
             ref[i] = acc
         assert_bits_equal(out.cpu().numpy(), ref, f"out nt={nt}")
         assert_bits_equal(got.cpu().numpy(), (resid.numpy() + ref).astype(np.float32), f"resid nt={nt}")
+
+
+@pytest.mark.parametrize("t,d,ff,E,k,nt", [(GType.Q8_0, 256, 256, 20, 16, 4097),    # 65552 pairs: also the fp32 hidden, not the Q8_0 rows
+                                           (GType.Q4_K, 8448, 256, 6, 2, 3)])        # d past 8192
+def test_sigmoid_decode_past_the_limits(cuda, t, d, ff, E, k, nt):
+    """MoeLayerRunner falls back to hy_moe_gate_up"""
+    L = layer(t, t, E, ff, d, seed=61)
+    rng = np.random.default_rng(62)
+    W_r = (rng.standard_normal((E, d)) * 0.05).astype(np.float32)
+    rb = rng.uniform(-0.05, 0.05, E).astype(np.float32)
+    dev = moe.MoeDev(L.to(cuda), torch.arange(E, dtype=torch.int32, device=cuda))
+    r = moe.MoeLayerRunner(dev, torch.from_numpy(W_r).to(cuda), k, max_rows=nt, router="sigmoid",
+                           router_bias=torch.from_numpy(rb).to(cuda))
+    x = torch.randn(nt, d, generator=gen(63))
+    out = r.decode(x.to(cuda)).clone()
+    torch.cuda.synchronize()
+    tok = np.arange(nt) if nt < 24 else np.r_[0, np.sort(rng.choice(nt, 22, replace=False)), nt - 1]
+    xs = x.numpy()[tok]
+    ids, wts, _ = orc.route_sig(r.logits.cpu().numpy()[tok, :E], rb, E, k, 1.0)
+    _, _, y = orc.moe_layer(oracle_layer(L), xs, ids, wts, want_hy=True)
+    y = (wts.reshape(-1, 1) * y).astype(np.float32).reshape(len(tok), k, d)
+    ref = np.zeros((len(tok), d), np.float32)
+    for i in range(len(tok)):
+        order = np.argsort(ids[i], kind="stable")
+        acc = y[i, order[0]].copy()
+        for j in order[1:]:
+            acc = (acc + y[i, j]).astype(np.float32)
+        ref[i] = acc
+    assert_bits_equal(out.cpu().numpy()[tok], ref, "out")
