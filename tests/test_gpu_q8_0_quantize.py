@@ -36,3 +36,23 @@ def test_routes_agree(cuda, n, nt, pad):
     if fin:
         ref = orc.quantize(GType.Q8_0, x[fin, :n].contiguous().numpy())
         np.testing.assert_array_equal(out[0].reshape(nt, -1)[fin], ref.reshape(len(fin), -1))
+
+
+def test_routes_agree_on_nan(cuda):
+    """NaN beside ordinary values, beside an infinity and alone in a block: the general kernel's bytes"""
+    n, nt = 96, 4
+    x = torch.randn(nt, n, generator=gen(72))
+    x[0, 5] = float("nan")
+    x[1, 32:64] = float("nan")
+    x[2, 64], x[2, 95] = float("inf"), float("nan")
+    x[3, ::4] = float("nan")          # one value of every lane
+    flat = torch.zeros(x.numel() + 4)
+    out = []
+    for off in (0, 1):
+        flat[off:off + x.numel()] = x.reshape(-1)
+        xd = flat.to(cuda)[off:]
+        q = torch.zeros(nt * q8_row_bytes(GType.Q8_0, n), dtype=torch.uint8, device=cuda)
+        moe.q8_quantize(GType.Q8_0, xd, n, n, nt, q)
+        torch.cuda.synchronize()
+        out.append(q.cpu().numpy())
+    np.testing.assert_array_equal(out[0], out[1])
