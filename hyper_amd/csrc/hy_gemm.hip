@@ -275,18 +275,17 @@ constexpr int GM_TOK = 64, GM_TILES = GM_TOK / 16, GM_ROWS = 64, GM_LD = 264;   
 __device__ __forceinline__ void store_f32(float *g, float v) { asm volatile("global_store_dword %0, %1, off" ::"v"(g), "v"(v) : "memory"); }
 
 // ------------------------------------------------------------------ the grouped GEMM stream
-// A block (8 waves, 512 threads, one per CU) owns 128 weight rows -- gate/up: 64 gate rows (waves 0-3) and the 64
-// up rows of the same outputs (waves 4-7); down: 128 rows -- and the work items blockIdx.y, + gridDim.y, ... (numbered
-// expert by expert, up to 64 tokens each).  Its steps, (item, 256-value span b) in order, form one stream.  Every
-// operand reaches LDS by DMA: a stage holds the 8 waves' 16-row weight tiles of span b (each one contiguous run of
-// the tiled layout) and the item's 64 activation rows of span b.  D stages rotate: step s computes from stage s % D
-// while the DMAs of steps s + 1 .. s + D - 1 are in flight.
+// A block of W waves owns 16 W weight rows -- gate/up: 8 W gate rows (the first half of the waves) and the up rows of the
+// same outputs; down: 16 W rows -- and the work items of its slot (up to 64 tokens of an expert each).  Its steps, (item,
+// 256-value span b) in order, form one stream.  Every operand reaches LDS by DMA: a stage holds the waves' 16-row weight
+// tiles of span b (each one contiguous run of the tiled layout) and the item's 64 activation rows of span b.  D stages
+// rotate: step s computes from stage s % D while the DMAs of steps s + 1 .. s + D - 1 are in flight.
 //
 // Waits are explicit.  Each wave issues the same L DMA instructions per step, and loads complete in issue order, so
-// "vmcnt <= (D - 2) L" right before issuing step s + D - 1 means this wave's step-s DMAs have landed; a barrier
-// then makes the whole stage visible and frees stage (s - 1) % D for the next issue.  Nothing in the stream is a
-// compiler-visible global load, so the compiler adds no waits of its own.  The epilogue's stores are not counted:
-// a store still in flight only makes a later wait stricter (loads cannot overtake the loads before them).
+// "vmcnt <= (D - 2) L" at the end of step s - 1, before step s + D - 1 is issued, means this wave's step-s DMAs have
+// landed; a barrier then makes the whole stage visible and frees stage (s - 1) % D for the next issue.  Nothing in the
+// stream is a compiler-visible global load, so the compiler adds no waits of its own.  The epilogue's stores are not
+// counted: a store still in flight only makes a later wait stricter (loads cannot overtake the loads before them).
 // Geometry of the stream kernel for weight type T, W waves (8 or 16) per block and B blocks per CU (1 or 2): the
 // stages get what is left of the CU's 160 KB LDS after the item tables.
 //
@@ -296,8 +295,9 @@ __device__ __forceinline__ void store_f32(float *g, float v) { asm volatile("glo
 // activation buffers: step s computes from weights s and aligned rows s while weights s + 1 and raw rows s + 2 are in
 // flight and rows s + 1 are copied; every wait is for all of a wave's DMAs.  509 tokens, 288 experts, d 4096, ff 1536,
 // top-8 in IQ4_NL: the layer call 2270 us with both operands staged through registers (k_gemm_nl: one step ahead, 4
-// waves, a 7-operation codebook and a 3-operation fold) -> 1038 us; bound by VALU issue (77 % of the cycles).  8 waves
-// of 32 rows instead of 16 of 16 share each activation read but hide less latency: 1196 against 1115 us at the time.
+// waves, a 7-operation codebook and a 3-operation fold) -> 1004 us; bound by VALU issue (71 and 75 % of the cycles of
+// gate/up and down).  8 waves of 32 rows instead of 16 of 16 share each activation read but hide less latency: 1196
+// against 1115 us at the time.
 template <int T, int W, int B> struct G5 {
     static constexpr bool A0 = vec_dot_type(T) == Q8_0;
     static constexpr int WAVES = W, THREADS = 64 * W, ROWS = 16 * W;   // a wave owns 16 weight rows
@@ -329,8 +329,8 @@ template <int T, int W, int B> struct G5 {
 // Q4_K and IQ4_XS gate/up (whose steps fit 128 registers): two blocks of 8 waves per CU, each block's stream running
 // independently of the other's; IQ2_XS, and Q6_K and IQ4_XS down: one block of 16 waves (256 weight rows share every
 // activation read; the steps fit 128 registers); the rest: one block of 8 waves (up to 256 registers, deeper rings).
-// IQ4_XS, the 1000-token layer call: 1185 us with 16 waves for both, 1125 as here, 1136 with 2 x 8 waves for both;
-// IQ2_XS: 3511 us with 16 waves, 3508 with 2 x 8.
+// IQ4_XS, the 1000-token layer call on one card: 1185 us with 16 waves for both, 1125 as here, 1136 with 2 x 8 waves for
+// both; IQ2_XS: 3511 us with 16 waves, 3508 with 2 x 8.  Small grids take 8 waves instead of 16: launch_k_gemm_fit.
 template <int T, bool GU> constexpr int g5_blocks() { return GU && (T == Q4_K || T == IQ4_XS) ? 2 : 1; }
 template <int T, bool GU> constexpr int g5_waves() { return T == IQ2_XS || (!GU && (T == Q6_K || T == IQ4_XS)) ? 16 : 8; }
 
@@ -508,7 +508,7 @@ __device__ __forceinline__ void step_q6k(const uint8_t *wt0, const int8_t *as, c
 // offset and not an addition.  It replaced the generic step (two masked 16x16x32 MFMAs a 32-value chunk, eight 24-bit
 // multiply-adds an output column, 8-byte codebook and sign rows): the 2048-token, 384-expert layer call of d 7168, ff
 // 2048, top-6: 6.29 -> 3.51 ms, and 3473 -> 3294 us with the plane table, the 16 : 1 split and the offsets (55 of 290
-// operations a wave and step less).  VALU issue and the LDS pipe bound it about alike.
+// operations a wave and step less).  Of the cycles VALU issue takes 64 %, the LDS pipe 58 %, the matrix cores 22 %.
 constexpr int IQ2_SEL = 512 + 128, IQ2_TAB = 4 * IQ2_SEL + 16 * 16;   // selectors (dwords); bytes with the plane table
 static_assert(IQ2_TAB % 256 == 0, "the stages behind it stay at multiples of 256");
 __device__ __forceinline__ void iq2_sel_table(uint32_t *sel) {
@@ -601,8 +601,8 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
 // group's lanes of B zeroed), si += scale D with 24-bit multiply-adds, the mins chained in an MFMA against the chunk's min.
 // Straight-line code per tile count; with one or two tiles the MFMAs of chunk c + 1 go out before chunk c is scaled.  (A
 // run-time tile loop took its branches at every chunk; without the empty asm on each sum the compiler regrouped the
-// chunks' sums and spilled.)  IQ4_XS, 1000 tokens, 288 experts, d 4096, ff 1536, top-8: the layer call 1252 -> 1125 us,
-// with the lds_at addresses and the geometry of g5_waves; bound by VALU issue (82 % of the cycles in gate/up).
+// chunks' sums and spilled.)  IQ4_XS, 1000 tokens, 288 experts, d 4096, ff 1536, top-8: the layer call 1252 -> 1125 us on
+// one card, with the lds_at addresses and the geometry of g5_waves; bound by VALU issue (82 % of the cycles in gate/up).
 // One tile of a type with 16-value groups (G1) leaves most of the 256 registers free and is bound by latency: its operand
 // reads go out together and its chunks are scheduled as one piece; with one chunk in flight at a time a layer call of 37
 // tokens (d 2048, 64 experts, ff 768, top-8) took 130.5 us in Q2_K, 133 in Q3_K and 141 in IQ2_S, here 124, 123 and 131
@@ -1175,7 +1175,7 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             }
             // the next step's stage has landed (this wave's DMAs; the barrier at its top covers the others'): waited for
             // here, ahead of the item's stores, so that no step waits for stores just issued (waited for at the next
-            // step's top: 131 MXFP4 tokens of 4096 x 2048, 8 experts, 116 us, here 113; 2048 Q5_K/Q6_K tokens 654, 645)
+            // step's top: 131 MXFP4 tokens, d 2048, 64 experts, ff 1024, top-8, 116 us, here 113; 2048 Q5_K/Q6_K tokens 654, 645)
             wait_vm<(D - 2) * C::L>();
             if (b != nsb - 1) return;
             // ---- the item's outputs, through this stage (every wave has finished reading it after a barrier), TOKP
@@ -1518,11 +1518,13 @@ static int cu_count() {
 }
 // item slots per row tile: enough blocks for about `per_cu` resident blocks on every CU.  k_gemm (`xcd`) groups its
 // slots by XCD when they are a multiple of 8, else places consecutive items P slots apart: from 8 slots up a
-// multiple of 8, else of P where there are that many.
+// multiple of 8, else of P where there are that many.  A multiple of 8 that leaves an eighth of the CUs without a block is
+// not worth its locality: 20 slots instead of 16 for 12 row blocks, 512 tokens (d 2048, 64 experts, ff 768, top-8) in
+// Q2_K 283 -> 252 us, in Q5_1 354 -> 314; the 509-token IQ4_NL call (288 experts) 1118 -> 1005.
 static int item_slots(int row_tiles, int n_pairs, int max_active, int per_cu, bool xcd = false) {
     const int want = cu_count() * per_cu / row_tiles;   // every block resident at once
     const int n = std::max(1, std::min(max_items(n_pairs, max_active), want));
-    if (xcd && n >= 8 && n / 8 * 8 * 8 > n * 7) return n / 8 * 8;   // (unless that would idle an eighth of the blocks)
+    if (xcd && n >= 8 && n / 8 * 8 * 8 > n * 7) return n / 8 * 8;
     const int P = 8 / xcd_gcd8(row_tiles);
     return n >= P ? n / P * P : n;
 }
