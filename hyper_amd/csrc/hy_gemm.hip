@@ -991,11 +991,11 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
     for (int seg = 0; seg < my_items; seg += C::ITEMS) {
         const int nit = min(C::ITEMS, my_items - seg);
         __syncthreads();   // readers of the previous segment's tables are done
-        // a thread id that the compiler cannot hoist out of the segment loop: kept live across the stream, the table
-        // addresses made from it went to scratch in the kernels near 128 registers (IQ4_NL, Q4_K gate/up), and a scratch
-        // reload is a vector memory operation that the compiler waits for by draining the stream
+        // IQ4_NL and Q4_K: a thread id that the compiler cannot hoist out of the segment loop.  Kept live across the stream,
+        // the table addresses made from it went to scratch there, and a scratch reload is a vector memory operation that
+        // the compiler waits for by draining the stream.
         int ts = tid;
-        asm volatile("" : "+v"(ts));
+        if constexpr (T == IQ4_NL || T == Q4_K) asm volatile("" : "+v"(ts));
         for (int i = ts; i < nit; i += C::THREADS) {
             const int k = seg + i;
             int pos = k * ys + ((k & 1) ? ys - 1 - y0 : y0);   // position in the class order
@@ -1190,9 +1190,9 @@ __global__ __launch_bounds__(64 * W, B * W / 4) void k_gemm(hy_moe_dev m, const 
             float *s_o = (float *) stage_w(stage);             // gate (or down) values
             float *s_u = s_o + TOKP * LD;                      // up values
             const int row0 = bx * OR;
-            // IQ4_NL is at its 128 registers: its epilogue makes its lane constants here instead of keeping them live across
-            // the stream (the other kernels have the registers, and are 1-3 % slower this way)
-            const int el = T == IQ4_NL ? lane_id_here() : lane, er = el & 15, eq = el >> 4;
+            // IQ4_NL and MXFP4 are at their 128 registers: the epilogue makes its lane constants here instead of keeping
+            // them live across the stream (the other kernels have the registers, and are 1-3 % slower this way)
+            const int el = T == IQ4_NL || T == MXFP4 ? lane_id_here() : lane, er = el & 15, eq = el >> 4;
             for (int p0 = 0; p0 < ntok; p0 += TOKP) {
                 lds_barrier();   // the stage (or the previous pass) is no longer read
                 {
