@@ -605,7 +605,7 @@ __device__ __forceinline__ void step_iq2xs(const uint8_t *wt0, const int8_t *as,
 // one card, with the lds_at addresses and the geometry of g5_waves; bound by VALU issue (82 % of the cycles in gate/up).
 // One tile of a type with 16-value groups (G1) leaves most of the 256 registers free and is bound by latency: its operand
 // reads go out together and its chunks are scheduled as one piece; with one chunk in flight at a time a layer call of 37
-// tokens (d 2048, 64 experts, ff 768, top-8) took 130.5 us in Q2_K, 133 in Q3_K and 141 in IQ2_S, here 124, 123 and 131
+// tokens (d 2048, 64 experts, ff 768, top-8) took 130.5 us in Q2_K, 133 in Q3_K and 141 in IQ2_S, here 125, 124 and 131
 // (the run-time tile loop: 120, 127 and 136).
 template <int T, int NT, bool FIRST>
 __device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, const int8_t *as, const float *yd, float (&acc)[GM_TILES][4]) {
@@ -619,7 +619,8 @@ __device__ __forceinline__ void step_gen(const uint8_t *wt, const uint2 *grid, c
     w.load(wt + rr * span_bytes(T), q);
     const uint32_t a0 = lds_addr(as) + rr * 256 + 16 * ((q >> 1) ^ rr) + 8 * (q & 1);   // row rr of tile 0, chunk 0
     const v4i z = {0, 0, 0, 0};
-    // (two tiles of 16-value groups, and one whose values come from a table: 141 instead of 131 us for IQ2_S as above)
+    // the MFMAs of chunk c + 1 ahead of chunk c's scaling: not for two tiles of 16-value groups (512 tokens in IQ2_S 241
+    // instead of 238 us) nor for one whose values come from a table in LDS (37 tokens in IQ2_S 139 instead of 131)
     constexpr int AHEAD = G ? G1 && !iq2_type(T) : NT <= 2;
     v4i D[1 + AHEAD][NT], E[1 + AHEAD][NT], sm[NT];
     int s0[1 + AHEAD], s1[1 + AHEAD], si[NT][4];
